@@ -29,6 +29,8 @@
  *   ndl_rms_norm        residual add + RMSNorm + weight product in one kernel
  *                       (qwen2.py:58-63, needle/layers/norm.py:14-17)
  *   ndl_silu_mul        silu(gate) * up of the SwiGLU MLP (needle/model/llama.py:36-37)
+ *   ndl_skinny_linear   a linear layer on up to 64 rows (a decode step's projections,
+ *   (+ _silu)           attention.py:84-96, llama.py:36-37)
  *   ndl_greedy_argmax   the greedy sampler's argmax for a batch of logit rows
  *                       (needle/model/sampler.py:27-28)
  *
@@ -379,6 +381,36 @@ int ndl_rms_norm(void* out, void* residual_out, const void* x, int64_t x_row_str
 int ndl_silu_mul(void* out, const void* gate, int64_t gate_row_stride, const void* up,
                  int64_t up_row_stride, int64_t rows, int intermediate, int dtype,
                  ndl_stream_t stream);
+
+/*
+ * A linear layer on few rows: out[r][c] = round(sum_k x[r][k] * weight[c][k] + bias[c]),
+ * fp32 products and sums, one rounding to the dtype (torch's F.linear).
+ *
+ * Replaces: the projections of needle/layers/attention.py:84-96 and needle/model/llama.py:36-37
+ *           on the rows of a decode step.
+ *
+ * out [rows][cols] and weight [cols][k] contiguous, x rows of k elements with row stride
+ * x_row_stride (a multiple of 8), bias [cols] or NULL; all 16-byte aligned.  Built for bf16
+ * and fp16, rows <= 64, cols a multiple of 16 (at most 2^28), k a multiple of 64 (k and
+ * x_row_stride at most 2^24): NDL_ERR_UNSUPPORTED otherwise.
+ */
+int ndl_skinny_linear(void* out, const void* x, int64_t x_row_stride, const void* weight,
+                      const void* bias, int rows, int cols, int k, int dtype,
+                      ndl_stream_t stream);
+
+/*
+ * The gate and up projections of the SwiGLU MLP and their product, on few rows:
+ *   out[r][c] = round(round(silu(g)) * u),
+ *   g = round(x[r] . weight[c]),  u = round(x[r] . weight[intermediate + c]),
+ * i.e. ndl_skinny_linear on the fused weight followed by ndl_silu_mul on its two halves.
+ *
+ * Replaces: needle/model/llama.py:36-37 (silu(gate_proj(x)) * up_proj(x)).
+ *
+ * weight [2 * intermediate][k] contiguous; out [rows][intermediate]; otherwise as
+ * ndl_skinny_linear with cols = intermediate.
+ */
+int ndl_skinny_linear_silu(void* out, const void* x, int64_t x_row_stride, const void* weight,
+                           int rows, int intermediate, int k, int dtype, ndl_stream_t stream);
 
 /*
  * Greedy sampling: out[r] = the index of the maximum of logits row r, in torch's argmax

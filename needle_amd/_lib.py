@@ -37,6 +37,8 @@ EXPORTED_SYMBOLS = (
     "ndl_kv_block_copy",
     "ndl_rms_norm",
     "ndl_silu_mul",
+    "ndl_skinny_linear",
+    "ndl_skinny_linear_silu",
     "ndl_greedy_argmax_workspace_bytes",
     "ndl_greedy_argmax",
 )
@@ -134,6 +136,14 @@ _SIGNATURES = {
     "ndl_silu_mul": (_c_i32, [
         _c_p, _c_p, _c_i64, _c_p, _c_i64,               # out, gate, stride, up, stride
         _c_i64, _c_i32, _c_i32, _c_p,                   # rows, intermediate, dtype, stream
+    ]),
+    "ndl_skinny_linear": (_c_i32, [
+        _c_p, _c_p, _c_i64, _c_p, _c_p,                 # out, x, stride, weight, bias
+        _c_i32, _c_i32, _c_i32, _c_i32, _c_p,           # rows, cols, k, dtype, stream
+    ]),
+    "ndl_skinny_linear_silu": (_c_i32, [
+        _c_p, _c_p, _c_i64, _c_p,                       # out, x, stride, weight
+        _c_i32, _c_i32, _c_i32, _c_i32, _c_p,           # rows, intermediate, k, dtype, stream
     ]),
     "ndl_greedy_argmax_workspace_bytes": (_c_sz, [_c_i64, _c_i32]),   # rows, vocab
     "ndl_greedy_argmax": (_c_i32, [

@@ -218,6 +218,59 @@ __device__ __forceinline__ float add_xor32(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// s_waitcnt vmcnt(N) with expcnt / lgkmcnt left unconstrained (gfx9 encoding:
+// vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] at bits 15:14).
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
+// Workgroup barrier without the vmcnt(0) drain __syncthreads() implies: callers wait
+// for exactly the loads they need first.  The memory clobber keeps the compiler from
+// moving LDS accesses across it.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
+// One direct global->LDS load: lane L reads 16 bytes at gbase + lane_off (gbase
+// wave-uniform) and they land at LDS byte address lds_addr + 16 * L (lds_addr uniform).
+// Issued from inline asm so the compiler does not order every later LDS read behind
+// it (it cannot tell the ring's stages apart); the ring waits on vmcnt itself.
+// M0 takes the LDS base; one wait state separates the M0 write from its use.  M0 is
+// a reserved register, so clang ignores it in the clobber list: this is sound only
+// while no other instruction in the kernels that use it keeps a value in M0, which
+// tests/test_isa_guards.py checks on the generated code.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void lds_dma16(const void* gbase, uint32_t lane_off,
+                                          uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(lane_off), "s"(gbase)
+               : "memory", "m0");
+}
+// The same for bytes that no other workgroup reads (streamed weights): nontemporal, so that
+// they do not displace what the caches are there for.
+__device__ __forceinline__ void lds_dma16_nt(const void* gbase, uint32_t lane_off,
+                                             uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(lane_off), "s"(gbase)
+               : "memory", "m0");
+}
+// The same with one dword per lane, landing at lds_addr + 4 * L.
+__device__ __forceinline__ void lds_dma4(const void* gbase, uint32_t lane_off, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(lane_off), "s"(gbase)
+               : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+// LDS byte address of a shared-memory pointer.
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+
 __device__ __forceinline__ u32x4 ldg16(const void* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
 }

@@ -3,8 +3,8 @@
 Same constructor, the same forward() signature and meaning
 (attention.py:36-96), the same parameter names (q_proj/k_proj/v_proj/o_proj),
 and the same KV pool layout [2, num_blocks, num_kv_heads, block_size,
-head_dim].  Projections stay torch GEMMs (attention.py:84-86); fuse_projections()
-runs the three as one GEMM over their concatenated weights.  The rest of
+head_dim].  Projections are torch GEMMs (attention.py:84-86), or ops.linear's kernel on the few
+rows of a decode step; fuse_projections() runs the three as one over their concatenated weights.  The rest of
 forward is, bit-exact with the reference's bf16 rounding of RoPE (attention.py:88,
 277-288):
 
@@ -36,16 +36,16 @@ import math
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from .. import ops
 from ..model.config import ModelConfig
+from .linear import Linear
 
 
 def fuse_linears(*mods: nn.Linear):
     """Puts the weights (and biases) of Linear layers that read the same input into one
     tensor, each layer's parameters becoming views of it, so that one GEMM serves them all
-    (F.linear over the fused weight, its output split).  Parameter names, values and
+    (ops.linear over the fused weight, its output split).  Parameter names, values and
     sharing with in-place updates are unchanged; the fused (weight, bias or None) is returned.
     Moving the layers afterwards gives them separate storage again, which fused_outputs
     detects."""
@@ -88,7 +88,7 @@ def fused_outputs(fused, mods, x):
     parameters are still views of it (fuse_linears), otherwise one per layer."""
     if fused is not None and _still_fused(fused, mods):
         w, b = fused
-        return F.linear(x, w, b).split([m.weight.shape[0] for m in mods], dim=-1)
+        return ops.linear(x, w, b).split([m.weight.shape[0] for m in mods], dim=-1)
     return tuple(m(x) for m in mods)
 
 
@@ -119,10 +119,10 @@ class Attention(nn.Module):
         self.head_dim = config.head_dim
         self.scale = 1.0 / math.sqrt(self.head_dim)
         hidden = config.hidden_size
-        self.q_proj = nn.Linear(hidden, self.num_heads * self.head_dim, bias=qkv_bias)
-        self.k_proj = nn.Linear(hidden, self.num_kv_heads * self.head_dim, bias=qkv_bias)
-        self.v_proj = nn.Linear(hidden, self.num_kv_heads * self.head_dim, bias=qkv_bias)
-        self.o_proj = nn.Linear(self.num_heads * self.head_dim, hidden, bias=False)
+        self.q_proj = Linear(hidden, self.num_heads * self.head_dim, bias=qkv_bias)
+        self.k_proj = Linear(hidden, self.num_kv_heads * self.head_dim, bias=qkv_bias)
+        self.v_proj = Linear(hidden, self.num_kv_heads * self.head_dim, bias=qkv_bias)
+        self.o_proj = Linear(self.num_heads * self.head_dim, hidden, bias=False)
         # Decode workspaces, newest last.  A grown workspace never frees the older ones: a
         # HIP graph captured with an older one keeps writing it on every replay.
         self._workspaces = []

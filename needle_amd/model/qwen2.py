@@ -19,7 +19,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
-from ..layers.attention import Attention, fuse_linears, fused_outputs
+from ..layers.attention import Attention, fuse_linears, fused_outputs, _still_fused
+from ..layers.linear import Linear
 from ..layers.norm import RMSNorm
 from ..layers.rope import RotaryEmbedding
 from .config import ModelConfig
@@ -28,9 +29,9 @@ from .config import ModelConfig
 class MLP(nn.Module):
     def __init__(self, config: ModelConfig):
         super().__init__()
-        self.gate_proj = nn.Linear(config.hidden_size, config.intermediate_size, bias=False)
-        self.up_proj = nn.Linear(config.hidden_size, config.intermediate_size, bias=False)
-        self.down_proj = nn.Linear(config.intermediate_size, config.hidden_size, bias=False)
+        self.gate_proj = Linear(config.hidden_size, config.intermediate_size, bias=False)
+        self.up_proj = Linear(config.hidden_size, config.intermediate_size, bias=False)
+        self.down_proj = Linear(config.intermediate_size, config.hidden_size, bias=False)
         self._gate_up = None   # fused gate/up projection (fuse_projections)
 
     def fuse_projections(self) -> None:
@@ -38,7 +39,12 @@ class MLP(nn.Module):
         self._gate_up = fuse_linears(self.gate_proj, self.up_proj)
 
     def forward(self, x):
-        gate, up = fused_outputs(self._gate_up, (self.gate_proj, self.up_proj), x)
+        mods = (self.gate_proj, self.up_proj)
+        if (self._gate_up is not None and ops.skinny_linear_takes(x, self._gate_up[0], None, 2)
+                and _still_fused(self._gate_up, mods)):
+            # a decode step: both projections and their product in one kernel
+            return self.down_proj(ops.linear_silu(x, self._gate_up[0]))
+        gate, up = fused_outputs(self._gate_up, mods, x)
         if x.is_cuda:   # one HIP kernel, torch's roundings
             shape = gate.shape
             act = ops.silu_mul(gate.reshape(-1, shape[-1]), up.reshape(-1, shape[-1]))
@@ -98,7 +104,7 @@ class CausalLM(nn.Module):
         super().__init__()
         self.config = config
         self.model = DecoderModel(config, qkv_bias)
-        self.lm_head = nn.Linear(config.hidden_size, config.vocab_size, bias=False)
+        self.lm_head = Linear(config.hidden_size, config.vocab_size, bias=False)
 
     def forward(self, input_ids, positions, kv_caches, block_table, cu_seqlens, context_lens,
                 max_seqlen, is_prefill):

@@ -88,3 +88,14 @@ def test_no_fused_fp16_multiply_add(device_asm, name):
         if m and m.group(6) != "0":
             bad.append(s)
     assert not bad, bad[:5]
+
+
+def test_skinny_linear_uses_m0_only_for_direct_lds_loads(device_asm):
+    body = [l.strip() for l in device_asm("skinny_linear")]
+    body = [l for l in body if l and not l.startswith((";", "."))]
+    uses = [i for i, l in enumerate(body) if re.search(r"\bm0\b", l)]
+    assert uses, "expected the direct-load M0 writes"
+    for i in uses:
+        assert body[i].startswith("s_mov_b32 m0, s"), body[i]
+        assert body[i + 1] == "s_nop 0" and \
+            re.match(r"global_load_lds_dwordx4 ", body[i + 2]), body[i:i + 3]
