@@ -43,14 +43,16 @@
 // arguments every format shares, then dispatch).
 #include <stdlib.h>
 
-#include "ndl_common.hpp"
+#include "decode_stream.hpp"
 
 namespace ndl {
 
-// The fewest tiles a wave of the automatic split takes: shorter pieces cost more in
-// partials and merge work than their parallelism gains (Llama-3-8B decode at one GPU's
-// share of 8-way tensor parallelism, 1 kv head, ~4.4 tiles per resident wave: 25.4 us per
-// layer at 5 tiles per wave, 23.3 at 8; shares with longer even splits are unchanged).
+// Empty stream slots before each sequence (see stream_slots), and the fewest slots a wave of
+// the automatic split takes: shorter pieces cost more in partials and merge work than their
+// parallelism gains (Llama-3-8B decode at one GPU's share of 8-way tensor parallelism, 1 kv
+// head, ~4.4 tiles per resident wave: 25.4 us per layer at 5 tiles per wave, 23.3 at 8; shares
+// with longer even splits are unchanged).
+constexpr int kStreamPad = 1;
 constexpr int kDecodeMinChunk = 8;
 // Waves per workgroup of the per-sequence split, and the most tiles per wave for which
 // the automatic choice takes it (a table of up to 256 columns at head_dim 64, 128 at
@@ -70,119 +72,6 @@ __device__ __forceinline__ typename VRow<D>::T load_vrow(const u16* p) {
     return ldg16(p);
   else
     return __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p));
-}
-
-struct DecodeArgs {
-  u16* out;
-  const u16* q;
-  int64_t q_tok_stride;
-  const u16* kplane;
-  const u16* vplane;
-  int64_t num_blocks;
-  int num_kv_heads;
-  const int32_t* block_table;
-  int64_t bt_row_stride;
-  int max_blocks;
-  // log2(block_size / 16): a block (table column) holds 1 << tile_shift tiles of 16 tokens;
-  // tile t of a sequence is rows 16 (t mod 2^shift) .. + 16 of its column t >> shift.
-  int tile_shift;
-  const int32_t* context_lens;
-  int num_heads;
-  int group;
-  float scale_log2;
-  int num_seqs;
-  int chunk;      // C: stream slots per wave; 0: ceil(T / waves) from the stream length T
-  int waves;      // waves per kv head
-  int nseg;       // segment slots per kv head: waves per kv head + num_seqs
-  float* ws_ml;   // [kv head][segment][group head][2] = (m, l)
-  float* ws_acc;  // [kv head][segment][group head][D]
-  // Fused append (null: none): the step's new k/v rows, [seq][kv head][D] with these token
-  // strides, written into the cache and attended in the same pass.
-  const u16* k_new;
-  const u16* v_new;
-  int64_t k_new_stride, v_new_stride;
-  // Rotary embedding of the step (null: q and k_new are already rotated): cos/sin rows of
-  // each sequence's new token, [seq][D] with row stride rope_stride.
-  const u16* rope_cos;
-  const u16* rope_sin;
-  int64_t rope_stride;
-};
-
-__device__ __forceinline__ int64_t attended_len(const DecodeArgs& a, int seq) {
-  int64_t L = (int64_t)a.context_lens[seq] + 1;  // attention.py:299
-  // a table row holds at most W blocks of 16 << tile_shift tokens
-  const int64_t cap = (int64_t)a.max_blocks << (4 + a.tile_shift);
-  return L < cap ? L : cap;
-}
-
-__device__ __forceinline__ int seq_tiles(const DecodeArgs& a, int q) {
-  const int64_t L = attended_len(a, q);
-  return L <= 0 ? 0 : (int)((L + 15) >> 4);
-}
-
-// Stream slots of a sequence with n tiles: kStreamPad empty slots, then its tiles (none for
-// a sequence with nothing to attend).  The empty slots stand for what a wave spends on
-// starting a sequence (its q rows, its table window and its first block load before any
-// tile computes), so that the waves that cross a sequence boundary take fewer tiles and
-// finish with the others.
-constexpr int kStreamPad = 1;
-__device__ __forceinline__ int stream_slots(int n) { return n > 0 ? n + kStreamPad : 0; }
-
-// Inclusive prefix sum over the 64 lanes of a wave.
-__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int o = __shfl_up(v, d, 64);
-    if (lane >= d) v += o;
-  }
-  return v;
-}
-
-// Stream position of sequence `target`'s first slot, or of the first sequence whose slots
-// reach past stream slot `tile` (target < 0).  Sequences are scanned 64 at a time; the scan
-// stops at the chunk that holds the answer.  Returns the sequence in *seq (num_seqs if none) and
-// its first slot in *first.
-__device__ __forceinline__ void stream_locate(const DecodeArgs& a, int lane, int target,
-                                              int64_t tile, int* seq, int64_t* first) {
-  int64_t carry = 0;
-  for (int base = 0; base < a.num_seqs; base += 64) {
-    const int q = base + lane;
-    const int n = q < a.num_seqs ? seq_tiles(a, q) : 0;
-    const int v = stream_slots(n);
-    const int incl = wave_incl_scan(v, lane);
-    const int64_t excl = carry + incl - v;
-    const uint64_t hit = target >= 0
-        ? __builtin_amdgcn_ballot_w64(q == target)
-        : __builtin_amdgcn_ballot_w64(q < a.num_seqs && n > 0 && excl + v > tile);
-    if (hit) {
-      const int l = __builtin_ctzll(hit);
-      *seq = base + l;
-      *first = __builtin_amdgcn_readlane((int)(excl - carry), l) + carry;
-      return;
-    }
-    carry += __builtin_amdgcn_readlane(incl, 63);
-  }
-  *seq = a.num_seqs;
-  *first = carry;
-}
-
-// Slots per wave: the fixed chunk, or the stream length (slots of all sequences of one
-// kv head) over the waves of a kv head, at least kDecodeMinChunk.
-// The chunk for a stream of `total` slots.
-__device__ __forceinline__ int64_t stream_chunk_of(const DecodeArgs& a, int64_t total) {
-  if (a.chunk > 0) return a.chunk;
-  const int64_t c = (total + a.waves - 1) / a.waves;
-  return c < kDecodeMinChunk ? kDecodeMinChunk : c;
-}
-__device__ __forceinline__ int64_t stream_chunk(const DecodeArgs& a, int lane) {
-  if (a.chunk > 0) return a.chunk;
-  int64_t total = 0;
-  for (int base = 0; base < a.num_seqs; base += 64) {
-    const int q = base + lane;
-    const int n = q < a.num_seqs ? seq_tiles(a, q) : 0;
-    total += __builtin_amdgcn_readlane(wave_incl_scan(stream_slots(n), lane), 63);
-  }
-  return stream_chunk_of(a, total);
 }
 
 // NW == 1: one wave per workgroup, wave s of a kv head takes stream slots s*C .. s*C + C.
@@ -575,7 +464,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
     int seq;
     if (one_load) {
       n_lane = lane < a.num_seqs ? seq_tiles(a, lane) : 0;
-      const int v_lane = stream_slots(n_lane);
+      const int v_lane = stream_slots<kStreamPad>(n_lane);
       const int incl = wave_incl_scan(v_lane, lane);
       const int total = __builtin_amdgcn_readlane(incl, 63);
       chunk = stream_chunk_of(a, total);
@@ -585,8 +474,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
       seq = hit ? __builtin_ctzll(hit) : a.num_seqs;
       first = hit ? __builtin_amdgcn_readlane(incl - v_lane, seq) : total;
     } else {
-      chunk = stream_chunk(a, lane);
-      stream_locate(a, lane, -1, (int64_t)sw * chunk, &seq, &first);
+      chunk = stream_chunk<kStreamPad>(a, lane);
+      stream_locate<kStreamPad>(a, lane, -1, (int64_t)sw * chunk, &seq, &first);
     }
     const int64_t start = (int64_t)sw * chunk, end = start + chunk;
     while (seq < a.num_seqs && first < end) {
@@ -598,7 +487,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
         if (s1 > s0)
           segment(seq, (int)(s0 - t0), (int)(s1 - t0), nt, sw + seq, nullptr);
       }
-      first += stream_slots(nt);
+      first += stream_slots<kStreamPad>(nt);
       ++seq;
     }
     if (held_seg >= 0) store_partial(held_seg, held, held_m, held_l);
@@ -666,160 +555,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(
         *reinterpret_cast<uint32_t*>(out_row) = w2[0];
     }
   }
-}
-
-// Merge of the segment partials: one wave per (query head, sequence).  A sequence
-// whose tiles lie in waves s0 .. s1 of its kv head's stream has its partials in
-// segment slots s0 + seq .. s1 + seq; a sequence inside one wave was written by the
-// attention kernel, and one with nothing to attend gets zeros here
-// (attention.py:307-308 on an empty context).
-// Pass 1 (lane-parallel over segments): global max, weights w_p = 2^(m_p - M)
-// into LDS, denominator sum_p w_p l_p.  Pass 2: sum_p w_p acc_p; the first
-// kMergePrefetch partials were loaded together with the (m, l) pairs, the rest
-// with independent, unrolled loads.
-constexpr int kMergeMaxParts = 2048;
-constexpr int kMergePrefetch = 8;
-
-template <int D, bool F16>
-__global__ __launch_bounds__(64) void paged_decode_merge_kernel(DecodeArgs a) {
-  constexpr int PER_LANE = D / 64;
-  __shared__ float wsh[kMergeMaxParts];
-  const int head = blockIdx.x, seq = blockIdx.y, lane = threadIdx.x;
-  const int kvh = head / a.group, hc = head - kvh * a.group;
-  // The decode step's new K/V row (ndl_paged_decode_append): the attention kernel attended
-  // it from registers; the first query head's wave of each (kv head, sequence) stores it,
-  // with the separate append's rule (attention.py:141-154): column min(ctx / bs, W - 1),
-  // row ctx % bs, nothing for a negative context or an invalid block id.
-  if (a.k_new != nullptr && hc == 0) {
-    constexpr int CH = D / 8;   // 16-byte chunks per row; lanes < CH: K, < 2 CH: V
-    const int ctx = a.context_lens[seq];
-    if (ctx >= 0 && lane < 2 * CH) {
-      const int bshift = 4 + a.tile_shift;   // log2(block_size)
-      const int pc = ctx >> bshift;
-      const int col = pc < a.max_blocks - 1 ? pc : a.max_blocks - 1;
-      const int64_t b = a.block_table[(int64_t)seq * a.bt_row_stride + col];
-      if (b >= 0 && b < a.num_blocks) {
-        const bool is_v = lane >= CH;
-        const int ch = is_v ? lane - CH : lane;
-        const u16* src_row = (is_v ? a.v_new + (int64_t)seq * a.v_new_stride
-                                   : a.k_new + (int64_t)seq * a.k_new_stride) + (int64_t)kvh * D;
-        u16* row = const_cast<u16*>(is_v ? a.vplane : a.kplane) +
-                   ((b * a.num_kv_heads + kvh) << bshift) * D +
-                   (int64_t)(ctx & ((1 << bshift) - 1)) * D + 8 * ch;
-        u32x4 val = ld16(src_row + 8 * ch);
-        if (!is_v && a.rope_cos != nullptr) {   // the key row rotated as the attention did
-          constexpr int HC = CH / 2;
-          const bool first_half = ch < HC;
-          const int lo_c = first_half ? ch : ch - HC;
-          const u32x4 partner = ld16(src_row + 8 * (ch ^ HC));
-          const u16* crow = a.rope_cos + (int64_t)seq * a.rope_stride + 8 * lo_c;
-          const u16* srow = a.rope_sin + (int64_t)seq * a.rope_stride + 8 * lo_c;
-          u32x4 lo, hi;
-          rope8<F16>(first_half ? val : partner, first_half ? partner : val, ld16(crow),
-                ld16(crow + 8 * HC), ld16(srow), ld16(srow + 8 * HC), lo, hi);
-          val = first_half ? lo : hi;
-        }
-        st16(row, val);
-      }
-    }
-  }
-  u16* dst = a.out + ((int64_t)seq * a.num_heads + head) * D + lane * PER_LANE;
-  // One pass over context_lens (one load per 64 sequences, nothing else in flight before
-  // it): this sequence's tiles, its first stream tile and the stream's total, i.e. what
-  // seq_tiles, stream_locate and stream_chunk give.
-  int nt = 0;
-  int64_t first = 0, total = 0;
-  for (int base = 0; base < a.num_seqs; base += 64) {
-    const int q = base + lane;
-    const int n = q < a.num_seqs ? seq_tiles(a, q) : 0;
-    const int v = stream_slots(n);
-    const int incl = wave_incl_scan(v, lane);
-    if (seq >= base && seq < base + 64) {   // the sequence's tile count and first tile
-      nt = __builtin_amdgcn_readlane(n, seq - base);
-      first = total + __builtin_amdgcn_readlane(incl - v, seq - base) + kStreamPad;
-    }
-    total += __builtin_amdgcn_readlane(incl, 63);
-  }
-  if (nt == 0) {
-    if constexpr (PER_LANE == 2)
-      *reinterpret_cast<uint32_t*>(dst) = 0u;
-    else
-      dst[0] = 0;
-    return;
-  }
-  const int64_t chunk = stream_chunk_of(a, total);
-  const int64_t s0 = first / chunk, s1 = (first + nt - 1) / chunk;
-  if (s0 == s1) return;
-  const int nparts = (int)(s1 - s0 + 1);
-  const int64_t slot0 = ((int64_t)kvh * a.nseg + s0 + seq) * a.group + hc;
-  const int64_t ml_stride = 2 * (int64_t)a.group, acc_stride = (int64_t)a.group * D;
-  const float* __restrict__ ml = a.ws_ml + slot0 * 2;
-  const float* __restrict__ src = a.ws_acc + slot0 * D + lane * PER_LANE;
-
-  // The first partials do not depend on the weights: load them with the (m, l) pairs.
-  float pre[kMergePrefetch][PER_LANE];
-#pragma unroll
-  for (int u = 0; u < kMergePrefetch; ++u)
-#pragma unroll
-    for (int e = 0; e < PER_LANE; ++e) pre[u][e] = u < nparts ? src[u * acc_stride + e] : 0.f;
-
-  // Part `lane`'s (m, l) pair (one 8-byte load) serves both passes below; parts from 64 on
-  // (a sequence over more than 64 stream waves) are read again in the second.
-  float m0 = kNegInf, l0 = 0.f;
-  if (lane < nparts) {
-    const float2 v = *reinterpret_cast<const float2*>(ml + lane * ml_stride);
-    m0 = v.x;
-    l0 = v.y;
-  }
-  float mx = m0;
-  for (int p = lane + 64; p < nparts; p += 64) mx = fmaxf(mx, ml[p * ml_stride]);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, xor_shfl(mx, o));
-  float den = 0.f;
-  if (lane < nparts) {
-    const float w = (m0 == kNegInf || mx == kNegInf) ? 0.f : fast_exp2(m0 - mx);
-    wsh[lane] = w;
-    den += w * l0;
-  }
-  for (int p = lane + 64; p < nparts; p += 64) {
-    const float mp = ml[p * ml_stride];
-    const float w = (mp == kNegInf || mx == kNegInf) ? 0.f : fast_exp2(mp - mx);
-    wsh[p] = w;
-    den += w * ml[p * ml_stride + 1];
-  }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) den += xor_shfl(den, o);
-  __syncthreads();
-
-  float acc[PER_LANE];
-#pragma unroll
-  for (int e = 0; e < PER_LANE; ++e) acc[e] = 0.f;
-#pragma unroll
-  for (int u = 0; u < kMergePrefetch; ++u)
-    if (u < nparts)
-#pragma unroll
-      for (int e = 0; e < PER_LANE; ++e) acc[e] += wsh[u] * pre[u][e];
-  int p = kMergePrefetch;
-  for (; p + 4 <= nparts; p += 4) {
-    float v[4][PER_LANE];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int e = 0; e < PER_LANE; ++e) v[u][e] = src[(p + u) * acc_stride + e];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int e = 0; e < PER_LANE; ++e) acc[e] += wsh[p + u] * v[u][e];
-  }
-  for (; p < nparts; ++p)
-#pragma unroll
-    for (int e = 0; e < PER_LANE; ++e) acc[e] += wsh[p] * src[p * acc_stride + e];
-
-  const float inv = den > 0.f ? 1.f / den : 0.f;
-  if constexpr (PER_LANE == 2)
-    *reinterpret_cast<uint32_t*>(dst) = Elt<F16>::pack(acc[0] * inv, acc[1] * inv);
-  else
-    dst[0] = Elt<F16>::one(acc[0] * inv);
 }
 
 // Blocks in flight per wave (2..4).  NDL_DECODE_DEPTH overrides the default for tuning.
@@ -1088,6 +823,7 @@ static int launch_decode(void* out, const void* q, int64_t q_tok_stride, const v
   a.scale_log2 = scale * kLog2e;
   a.num_seqs = num_seqs;
   a.chunk = (int)lay.chunk;
+  a.min_chunk = kDecodeMinChunk;
   a.waves = (int)lay.waves;
   a.nseg = (int)lay.nseg;
   a.ws_ml = (float*)workspace;
@@ -1120,14 +856,8 @@ static int launch_decode(void* out, const void* q, int64_t q_tok_stride, const v
   }
   int rc = check_launch();
   if (rc != NDL_OK) return rc;
-  const dim3 mgrid((unsigned)num_heads, (unsigned)num_seqs);
-  if (head_dim == 128)
-    hipLaunchKernelGGL((f16 ? paged_decode_merge_kernel<128, true>
-                            : paged_decode_merge_kernel<128, false>), mgrid, dim3(64), 0, s, a);
-  else
-    hipLaunchKernelGGL((f16 ? paged_decode_merge_kernel<64, true>
-                            : paged_decode_merge_kernel<64, false>), mgrid, dim3(64), 0, s, a);
-  return check_launch();
+  return f16 ? launch_decode_merge<kFmtF16, kStreamPad>(a, head_dim, s)
+             : launch_decode_merge<kFmtBF16, kStreamPad>(a, head_dim, s);
 }
 
 }  // namespace ndl
