@@ -164,6 +164,35 @@ size_t ndl_paged_decode_workspace_bytes(int num_seqs, int num_heads, int num_kv_
                                         int partition_tokens);
 
 /*
+ * Bytes of scratch ndl_paged_decode_f32 splits long sequences with (a fixed function of the
+ * arguments and the device, 0 for an invalid shape).
+ */
+size_t ndl_paged_decode_f32_workspace_bytes(int num_seqs, int num_heads, int num_kv_heads,
+                                            int head_dim, int max_blocks_per_seq,
+                                            int block_size);
+
+/*
+ * The decode step in float32 with its work split over the whole GPU: what ndl_paged_decode
+ * (k, v, cos and sin NULL), ndl_paged_decode_append (cos and sin NULL) or
+ * ndl_rope_paged_decode_append give for NDL_DTYPE_F32, up to the order of the fp32 sums.  With
+ * a 16-byte aligned workspace of ndl_paged_decode_f32_workspace_bytes (calls that share one
+ * must not overlap) sequences are split over workgroups and merged; with none, or a smaller
+ * one, each (kv head, sequence) is one workgroup, as in those entry points.
+ *
+ * Replaces: needle/layers/attention.py:140-159, :291-310 in a float32 model.
+ */
+int ndl_paged_decode_f32(void* out, const void* q, int64_t q_tok_stride,
+                         const void* k, int64_t k_tok_stride,
+                         const void* v, int64_t v_tok_stride,
+                         const void* cos, const void* sin, int64_t cs_tok_stride,
+                         void* kv_cache, int64_t num_blocks,
+                         const int32_t* block_table, int64_t bt_row_stride,
+                         int max_blocks_per_seq, const int32_t* context_lens, int num_seqs,
+                         int num_heads, int num_kv_heads, int head_dim, int block_size,
+                         float scale, void* workspace, size_t workspace_bytes,
+                         ndl_stream_t stream);
+
+/*
  * Paged decode attention, one query token per sequence.
  *
  * Replaces: needle/layers/attention.py:291-310 (_decode_pytorch) and the

@@ -28,6 +28,8 @@ EXPORTED_SYMBOLS = (
     "ndl_kv_append",
     "ndl_rope_kv_append",
     "ndl_paged_decode_workspace_bytes",
+    "ndl_paged_decode_f32_workspace_bytes",
+    "ndl_paged_decode_f32",
     "ndl_paged_decode",
     "ndl_paged_decode_append",
     "ndl_paged_decode_append_noalloc",
@@ -67,6 +69,17 @@ _SIGNATURES = {
         _c_p, _c_p, _c_i32, _c_i64, _c_p,               # cu, ctx, B, T, stream
     ]),
     "ndl_paged_decode_workspace_bytes": (_c_sz, [_c_i32] * 7),
+    "ndl_paged_decode_f32_workspace_bytes": (_c_sz, [_c_i32] * 6),
+    "ndl_paged_decode_f32": (_c_i32, [
+        _c_p, _c_p, _c_i64,                             # out, q, q stride
+        _c_p, _c_i64, _c_p, _c_i64,                     # k, k stride, v, v stride
+        _c_p, _c_p, _c_i64,                             # cos, sin, cos/sin stride
+        _c_p, _c_i64,                                   # cache, NB
+        _c_p, _c_i64, _c_i32,                           # block_table, row stride, W
+        _c_p, _c_i32,                                   # ctx, B
+        _c_i32, _c_i32, _c_i32, _c_i32,                 # H, Hkv, D, bs
+        _c_f32, _c_p, _c_sz, _c_p,                      # scale, workspace, bytes, stream
+    ]),
     "ndl_paged_decode": (_c_i32, [
         _c_p, _c_p, _c_i64,                             # out, q, q stride
         _c_p, _c_i64,                                   # cache, NB

@@ -326,15 +326,18 @@ int launch_kv_append(void* kv_cache, int64_t num_blocks, int num_kv_heads, int b
 
 // The float32 attention launchers (paged_decode_f32.hip, varlen_prefill_f32.hip); the entry
 // points check the arguments common to all formats first.  k_new/v_new non-null: the step's
-// rows are appended first (by ndl_kv_append's kernel); cos/sin non-null: q (and k_new) are
-// rotated.
+// rows are attended and stored; cos/sin non-null: q (and k_new) are rotated.  A workspace of
+// decode_f32_workspace_bytes lets the decode split sequences over workgroups; without one, or
+// with a smaller one, it takes one workgroup per (kv head, sequence).
 int launch_decode_f32(void* out, const void* q, int64_t q_tok_stride, const void* k_new,
                       int64_t k_tok_stride, const void* v_new, int64_t v_tok_stride,
                       const void* cos, const void* sin, int64_t cs_tok_stride, void* kv_cache,
                       int64_t num_blocks, const int32_t* block_table, int64_t bt_row_stride,
                       int max_blocks_per_seq, const int32_t* context_lens, int num_seqs,
                       int num_heads, int num_kv_heads, int head_dim, int block_size, float scale,
-                      ndl_stream_t stream);
+                      void* workspace, size_t workspace_bytes, ndl_stream_t stream);
+size_t decode_f32_workspace_bytes(int num_seqs, int num_heads, int num_kv_heads, int head_dim,
+                                  int64_t max_tiles);
 int launch_prefill_f32(void* out, const void* q, int64_t q_tok_stride, const void* cos,
                        const void* sin, int64_t cs_tok_stride, const void* kv_cache,
                        int64_t num_blocks, const int32_t* block_table, int64_t bt_row_stride,

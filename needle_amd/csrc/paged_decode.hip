@@ -698,6 +698,18 @@ extern "C" size_t ndl_paged_decode_workspace_bytes(int num_seqs, int num_heads, 
   return lay.bytes;
 }
 
+extern "C" size_t ndl_paged_decode_f32_workspace_bytes(int num_seqs, int num_heads,
+                                                       int num_kv_heads, int head_dim,
+                                                       int max_blocks_per_seq, int block_size) {
+  using namespace ndl;
+  const int tshift = block_tile_shift(block_size);
+  if (num_seqs <= 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 ||
+      (head_dim != 64 && head_dim != 128) || max_blocks_per_seq <= 0 || tshift < 0)
+    return 0;
+  return decode_f32_workspace_bytes(num_seqs, num_heads, num_kv_heads, head_dim,
+                                    (int64_t)max_blocks_per_seq << tshift);
+}
+
 namespace ndl {
 
 // Allocation-free decode (ndl_paged_decode_append_noalloc): the split-K partials go to a
@@ -754,7 +766,8 @@ static int launch_decode(void* out, const void* q, int64_t q_tok_stride, const v
                          size_t workspace_bytes, const void* k_new, int64_t k_new_stride,
                          const void* v_new, int64_t v_new_stride, ndl_stream_t stream,
                          bool static_scratch = false, const void* rope_cos = nullptr,
-                         const void* rope_sin = nullptr, int64_t rope_stride = 0) {
+                         const void* rope_sin = nullptr, int64_t rope_stride = 0,
+                         bool f32_workspace = false) {
   if (!dtype_known(dtype)) return NDL_ERR_UNSUPPORTED;
   const int tshift = block_tile_shift(block_size);
   if (tshift < 0 || (head_dim != 64 && head_dim != 128)) return NDL_ERR_UNSUPPORTED;
@@ -774,14 +787,16 @@ static int launch_decode(void* out, const void* q, int64_t q_tok_stride, const v
   if (num_seqs > 65535) return NDL_ERR_UNSUPPORTED;
   if (dtype_is_f32(dtype)) {
     // One workgroup per (kv head, sequence) whatever the split asks for (the values are
-    // checked as for the other formats); no partials, so neither workspace nor scratch.
+    // checked as for the other formats) unless the caller passed a workspace for it
+    // (ndl_paged_decode_f32): no partials, so neither workspace nor scratch.
     if (partition_tokens < -1 || (partition_tokens > 0 && partition_tokens % 16 != 0))
       return NDL_ERR_INVALID_ARG;
     return launch_decode_f32(out, q, q_tok_stride, k_new, k_new_stride, v_new, v_new_stride,
                              rope_cos, rope_sin, rope_stride, const_cast<void*>(kv_cache),
                              num_blocks, block_table, bt_row_stride, max_blocks_per_seq,
                              context_lens, num_seqs, num_heads, num_kv_heads, head_dim,
-                             block_size, scale, stream);
+                             block_size, scale, f32_workspace ? workspace : nullptr,
+                             workspace_bytes, stream);
   }
   DecodeLayout lay;
   const int64_t max_tiles = (int64_t)max_blocks_per_seq << tshift;
@@ -887,7 +902,8 @@ static int launch_decode_append(void* out, const void* q, int64_t q_tok_stride, 
                                 float scale, int partition_tokens, void* workspace,
                                 size_t workspace_bytes, ndl_stream_t stream,
                                 bool static_scratch, const void* rope_cos = nullptr,
-                                const void* rope_sin = nullptr, int64_t rope_stride = 0) {
+                                const void* rope_sin = nullptr, int64_t rope_stride = 0,
+                                bool f32_workspace = false) {
   if (num_seqs > 0) {
     if (!k || !v) return NDL_ERR_INVALID_ARG;
     if (rope_cos != nullptr || rope_sin != nullptr) {
@@ -904,7 +920,7 @@ static int launch_decode_append(void* out, const void* q, int64_t q_tok_stride, 
                        max_blocks_per_seq, context_lens, num_seqs, num_heads, num_kv_heads,
                        head_dim, block_size, dtype, scale, partition_tokens, workspace,
                        workspace_bytes, k, k_tok_stride, v, v_tok_stride, stream,
-                       static_scratch, rope_cos, rope_sin, rope_stride);
+                       static_scratch, rope_cos, rope_sin, rope_stride, f32_workspace);
 }
 
 }  // namespace ndl
@@ -954,4 +970,30 @@ extern "C" int ndl_rope_paged_decode_append(
                                    num_kv_heads, head_dim, block_size, dtype, scale,
                                    partition_tokens, workspace, workspace_bytes, stream, false,
                                    cos, sin, cs_tok_stride);
+}
+
+// float32 with a workspace for the split of long sequences.
+extern "C" int ndl_paged_decode_f32(void* out, const void* q, int64_t q_tok_stride, const void* k,
+                                    int64_t k_tok_stride, const void* v, int64_t v_tok_stride,
+                                    const void* cos, const void* sin, int64_t cs_tok_stride,
+                                    void* kv_cache, int64_t num_blocks,
+                                    const int32_t* block_table, int64_t bt_row_stride,
+                                    int max_blocks_per_seq, const int32_t* context_lens,
+                                    int num_seqs, int num_heads, int num_kv_heads, int head_dim,
+                                    int block_size, float scale, void* workspace,
+                                    size_t workspace_bytes, ndl_stream_t stream) {
+  if (k == nullptr && v == nullptr) {
+    if (cos != nullptr || sin != nullptr) return NDL_ERR_INVALID_ARG;
+    return ndl::launch_decode(out, q, q_tok_stride, kv_cache, num_blocks, block_table,
+                              bt_row_stride, max_blocks_per_seq, context_lens, num_seqs,
+                              num_heads, num_kv_heads, head_dim, block_size, NDL_DTYPE_F32,
+                              scale, 0, workspace, workspace_bytes, nullptr, 0, nullptr, 0,
+                              stream, false, nullptr, nullptr, 0, true);
+  }
+  return ndl::launch_decode_append(out, q, q_tok_stride, k, k_tok_stride, v, v_tok_stride,
+                                   kv_cache, num_blocks, block_table, bt_row_stride,
+                                   max_blocks_per_seq, context_lens, num_seqs, num_heads,
+                                   num_kv_heads, head_dim, block_size, NDL_DTYPE_F32, scale, 0,
+                                   workspace, workspace_bytes, stream, false, cos, sin,
+                                   cs_tok_stride, true);
 }

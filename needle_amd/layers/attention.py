@@ -180,7 +180,8 @@ class Attention(nn.Module):
     def _decode_attend(self, q, kv_cache, block_table, context_lens, new_k=None, new_v=None,
                        cos=None, sin=None):
         need = ops.decode_workspace_bytes(q.shape[0], self.num_heads, self.num_kv_heads,
-                                          self.head_dim, block_table.shape[1], kv_cache.shape[3])
+                                          self.head_dim, block_table.shape[1], kv_cache.shape[3],
+                                          dtype=q.dtype)
         ws = self._workspaces[-1] if self._workspaces else None
         if ws is None or ws.numel() < need or ws.device != q.device:
             ws = ops.decode_workspace(need, q.device)

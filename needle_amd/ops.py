@@ -217,7 +217,12 @@ def write_kv(k, v, kv_cache, block_table, cu_seqlens, context_lens) -> None:
 
 def decode_workspace_bytes(num_seqs: int, num_heads: int, num_kv_heads: int, head_dim: int,
                            max_blocks_per_seq: int, block_size: int = 16,
-                           partition_tokens: int = 0) -> int:
+                           partition_tokens: int = 0, dtype: Optional[torch.dtype] = None) -> int:
+    """Bytes of the workspace paged_decode uses for this shape (dtype: of the pool; float32's
+    split has a size of its own)."""
+    if dtype == torch.float32 and partition_tokens == 0:
+        return int(_lib.load().ndl_paged_decode_f32_workspace_bytes(
+            num_seqs, num_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size))
     return int(_lib.load().ndl_paged_decode_workspace_bytes(
         num_seqs, num_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size,
         partition_tokens))
@@ -271,13 +276,26 @@ def paged_decode(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Ten
         _validate_slots(block_table, num_blocks)
     lib = _lib.load()
     w = block_table.shape[1]
-    need = int(lib.ndl_paged_decode_workspace_bytes(
-        n_seqs, num_heads, num_kv_heads, head_dim, w, bs, partition_tokens))
+    need = decode_workspace_bytes(n_seqs, num_heads, num_kv_heads, head_dim, w, bs,
+                                  partition_tokens, q.dtype)
     _require(need > 0, "unsupported decode shape")
     if workspace is None or workspace.numel() * workspace.element_size() < need:
         workspace = decode_workspace(need, dev)
+    f32_split = q.dtype == torch.float32 and partition_tokens == 0
+
+    def decode_f32(ks=0, vs=0, cs=0):
+        rc = lib.ndl_paged_decode_f32(
+            out.data_ptr(), q.data_ptr(), qs, _ptr(new_k), ks, _ptr(new_v), vs, _ptr(cos),
+            _ptr(sin), cs, kv_cache.data_ptr(), num_blocks, block_table.data_ptr(),
+            block_table.stride(0), w, context_lens.data_ptr(), n_seqs, num_heads, num_kv_heads,
+            head_dim, bs, float(scale), workspace.data_ptr(), need, _stream(dev))
+        _lib.check(rc, "ndl_paged_decode_f32")
+        return out
+
     if new_k is None and new_v is None:
         _require(cos is None and sin is None, "cos / sin need new_k / new_v")
+        if f32_split:
+            return decode_f32()
         rc = lib.ndl_paged_decode(
             out.data_ptr(), q.data_ptr(), qs, kv_cache.data_ptr(), num_blocks,
             block_table.data_ptr(), block_table.stride(0), w,
@@ -301,6 +319,8 @@ def paged_decode(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Ten
             _require(x.device == dev and x.stride(1) == 1, f"{name} rows must be contiguous")
         _require(cos.stride(0) == sin.stride(0) or n_seqs <= 1, "cos and sin strides differ")
         cs = cos.stride(0) if n_seqs > 1 else head_dim
+        if f32_split:
+            return decode_f32(ks, vs, cs)
         rc = lib.ndl_rope_paged_decode_append(
             out.data_ptr(), q.data_ptr(), qs, new_k.data_ptr(), ks, new_v.data_ptr(), vs,
             cos.data_ptr(), sin.data_ptr(), cs,
@@ -310,6 +330,8 @@ def paged_decode(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Ten
             _stream(dev))
         _lib.check(rc, "ndl_rope_paged_decode_append")
         return out
+    if f32_split:
+        return decode_f32(ks, vs)
     rc = lib.ndl_paged_decode_append(
         out.data_ptr(), q.data_ptr(), qs, new_k.data_ptr(), ks, new_v.data_ptr(), vs,
         kv_cache.data_ptr(), num_blocks, block_table.data_ptr(), block_table.stride(0), w,
