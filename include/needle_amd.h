@@ -352,6 +352,32 @@ int ndl_rope_varlen_prefill(void* out, const void* q, int64_t q_tok_stride,
                             float scale, ndl_stream_t stream);
 
 /*
+ * The same prefill attention (cos and sin NULL: ndl_varlen_prefill, otherwise
+ * ndl_rope_varlen_prefill) with a workspace of ndl_varlen_prefill_workspace_bytes, 16-byte
+ * aligned (calls that share one must not overlap): where few query tiles attend many keys
+ * (a prompt after a long cached prefix, one long prompt), the keys of each tile are split over
+ * workgroups and the pieces merged, in two launches.  Results differ by the order of the fp32
+ * sums.  workspace NULL or too small, or a shape of 0 bytes: as those entry points.
+ *
+ * Replaces: needle/layers/attention.py:120-134 (_prefill_pytorch).
+ */
+#define NDL_PREFILL_SPLIT_MIN_KEYS 768   /* 0 bytes for tables of fewer tokens per row */
+size_t ndl_varlen_prefill_workspace_bytes(int num_seqs, int64_t num_tokens, int max_seqlen,
+                                          int max_blocks_per_seq, int num_heads,
+                                          int num_kv_heads, int head_dim, int block_size,
+                                          int dtype);
+int ndl_varlen_prefill_split(void* out, const void* q, int64_t q_tok_stride,
+                             const void* cos, const void* sin, int64_t cs_tok_stride,
+                             const void* kv_cache, int64_t num_blocks,
+                             const int32_t* block_table, int64_t bt_row_stride,
+                             int max_blocks_per_seq, const int32_t* cu_seqlens,
+                             const int32_t* context_lens, int num_seqs, int64_t num_tokens,
+                             int max_seqlen, int max_context_len,
+                             int num_heads, int num_kv_heads, int head_dim, int block_size,
+                             int dtype, float scale, void* workspace, size_t workspace_bytes,
+                             ndl_stream_t stream);
+
+/*
  * Copy whole KV blocks between two sets of per-layer pools: the swap-out (GPU pool ->
  * pinned CPU pool) and swap-in (CPU pool -> GPU pool) copies of a preemption.
  *

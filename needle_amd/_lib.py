@@ -17,6 +17,7 @@ LIB_PATH = _PKG_DIR / "libneedle_amd.so"
 
 NDL_ABI_VERSION = 8
 NDL_DECODE_STATIC_SCRATCH_BYTES = 16 << 20
+NDL_PREFILL_SPLIT_MIN_KEYS = 768
 NDL_DTYPE_BF16 = 0
 NDL_DTYPE_F16 = 1
 NDL_DTYPE_F32 = 2
@@ -36,6 +37,8 @@ EXPORTED_SYMBOLS = (
     "ndl_rope_paged_decode_append",
     "ndl_varlen_prefill",
     "ndl_rope_varlen_prefill",
+    "ndl_varlen_prefill_workspace_bytes",
+    "ndl_varlen_prefill_split",
     "ndl_kv_block_copy",
     "ndl_rms_norm",
     "ndl_silu_mul",
@@ -135,6 +138,16 @@ _SIGNATURES = {
         _c_p, _c_p, _c_i32, _c_i64, _c_i32, _c_i32,     # cu, ctx, B, T, max_seqlen, max_ctx
         _c_i32, _c_i32, _c_i32, _c_i32, _c_i32,         # H, Hkv, D, bs, dtype
         _c_f32, _c_p,                                   # scale, stream
+    ]),
+    "ndl_varlen_prefill_workspace_bytes": (_c_sz, [_c_i32, _c_i64] + [_c_i32] * 7),
+    "ndl_varlen_prefill_split": (_c_i32, [
+        _c_p, _c_p, _c_i64,                             # out, q, q stride
+        _c_p, _c_p, _c_i64,                             # cos, sin, cos/sin stride
+        _c_p, _c_i64,                                   # cache, NB
+        _c_p, _c_i64, _c_i32,                           # block_table, row stride, W
+        _c_p, _c_p, _c_i32, _c_i64, _c_i32, _c_i32,     # cu, ctx, B, T, max_seqlen, max_ctx
+        _c_i32, _c_i32, _c_i32, _c_i32, _c_i32,         # H, Hkv, D, bs, dtype
+        _c_f32, _c_p, _c_sz, _c_p,                      # scale, workspace, bytes, stream
     ]),
     "ndl_kv_block_copy": (_c_i32, [
         _c_p, _c_i64, _c_p, _c_i64,                     # dst pools, dst NB, src pools, src NB

@@ -51,6 +51,11 @@ constexpr int kPrefWaves = 8;          // waves (jobs) per workgroup
 // Tile-list limits of the persistent launch (larger batches use one workgroup per tile).
 constexpr int kPrefListSeqs = 8192;
 constexpr int kPrefListLevels = 2048;
+// The split launch: most (sequence, query tile) pairs of its plan, the empty slots before each
+// tile (what a tile's start costs in steps), and the fewest slots a workgroup takes.
+constexpr int kPrefSplitTiles = 1024;
+constexpr int kPrefPad = 4;
+constexpr int kPrefMinSteps = 16;
 // exp2-domain growth of a row max tolerated before the accumulator is rescaled:
 // probabilities stay <= 2^8, exact in bf16's exponent range and in fp32 sums.
 constexpr float kRescaleSlack = 8.0f;
@@ -85,6 +90,11 @@ struct PrefillArgs {
   const u16* rope_cos;
   const u16* rope_sin;
   int64_t rope_stride;
+  // The split launch: workgroups per kv head and its workspace.
+  int takers;
+  int32_t* ws_plan;   // [2 + tiles]: C, tiles, stream slot of each tile's first step
+  float* ws_ml;       // [slot][wave][lane][2] = (m, l)
+  float* ws_acc;      // [slot][wave][accumulator quad][lane][4]
 };
 
 // One workgroup tile, looked up one tile ahead by the persistent walk: jobs
@@ -94,6 +104,8 @@ struct PrefillArgs {
 struct PrefTile {
   int seq, qtile, kvh;
   int tok0, tok1, ctx;
+  int sb, se;   // steps taken: sb .. se (the split launch; se past the last step otherwise)
+  int slot;     // where a piece of the tile's steps leaves its partial; < 0: it has them all
 };
 
 typedef __attribute__((ext_vector_type(4))) short i16x4v;
@@ -138,8 +150,9 @@ __device__ __forceinline__ float half_sum(float v) {
 // ROPE: q is the raw projection; each Q row is rotated as it is read into the operand
 // registers (with the reference's rounding, rope8), from cos/sin rows of its token.
 // F16: the elements are fp16 (else bf16).
-template <int D, int NS, bool ROPE, bool F16>
-__global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(PrefillArgs a) {
+// SPLIT: the launch of prefill_split_kernel (below).
+template <int D, int NS, bool ROPE, bool F16, bool SPLIT>
+__device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
   using T = Elt<F16>;
   using X8 = typename T::x8;
   constexpr int KS = D / 16;          // k-steps of the QK MFMA (16 head_dim each)
@@ -176,7 +189,7 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
   typedef const __attribute__((address_space(4))) int32_t* cptr;
   auto look_up = [&](int seq, int qtile, int kvh) {
     const cptr cu = (cptr)a.cu_seqlens, cl = (cptr)a.context_lens;
-    return PrefTile{seq, qtile, kvh, cu[seq], cu[seq + 1], cl[seq]};
+    return PrefTile{seq, qtile, kvh, cu[seq], cu[seq + 1], cl[seq], 0, 0x7fffffff, -1};
   };
   // First row of a tile's first job.
   auto first_row = [&](int qtile) { return qtile * kPrefWaves / a.group * kPrefRows; };
@@ -215,7 +228,10 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
     const int row0 = job0 / a.group * kPrefRows;                 // the tile's first row
     const int row_end = ((job0 + kPrefWaves - 1) / a.group + 1) * kPrefRows;
     const int kv_end = ctx + (row_end < n ? row_end : n);
-    const int nsteps = (kv_end + kPrefKeys - 1) / kPrefKeys;
+    // Steps count from the first one taken, step0 of the tile (0 unless SPLIT).
+    const int all_steps = (kv_end + kPrefKeys - 1) / kPrefKeys;
+    const int step0 = SPLIT ? t.sb : 0;
+    const int nsteps = (SPLIT && t.se < all_steps ? t.se : all_steps) - step0;
 
     const int wrow0 = sub * kPrefRows;                           // first row of this wave
     const bool wave_active = wrow0 < n;
@@ -239,7 +255,7 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
     // readlane (uniform).  The first window goes out with the Q loads below and one wait
     // covers both; a later refill waits for every outstanding load (a vector-memory wait
     // cannot single one out); it happens once per 64 tiles.
-    int win0 = 0;
+    int win0 = SPLIT ? (2 * step0) & ~63 : 0;
     int btw = 0;
     uint64_t win_badm = 0;
     auto to_unit = [&](int raw, int t) {
@@ -248,7 +264,8 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
     };
     if (!pre && wave == 0) {
       const int l = fresh_lane();
-      lds_dma4(bt_row, 4u * (uint32_t)((l < a.max_tiles ? l : a.max_tiles - 1) >> tshift),
+      const int w = (SPLIT ? win0 : 0) + l;
+      lds_dma4(bt_row, 4u * (uint32_t)((w < a.max_tiles ? w : a.max_tiles - 1) >> tshift),
                lds_addr(s_btw));
       vm_wait<0>();
     }
@@ -297,7 +314,7 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
     // rows past the range read whatever the table maps them to.  The softmax masks both.
     // A window of the table with no invalid id (the normal case) sets no bits.
     auto stage_in = [&](int step, int stage) {
-      const int c0 = clamp_col(2 * step), c1 = clamp_col(2 * step + 1);  // same 64-window
+      const int c0 = clamp_col(2 * (step0 + step)), c1 = clamp_col(2 * (step0 + step) + 1);  // same 64-window
       if (c0 < win0 || c0 >= win0 + 64) {
         win0 = c0 & ~63;
         const int l = fresh_lane();
@@ -417,10 +434,10 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
     // its loads have landed (one barrier before its PV).  Only a workgroup's last step
     // and steps over invalid block ids need this.
     auto needs_vzero = [&](int step, int stage) {
-      return step * kPrefKeys + kPrefKeys > kv_end || ((badbits >> (2 * stage)) & 3u) != 0;
+      return (step0 + step) * kPrefKeys + kPrefKeys > kv_end || ((badbits >> (2 * stage)) & 3u) != 0;
     };
     auto zero_v = [&](int step, int stage) {
-      const int kv0 = step * kPrefKeys;
+      const int kv0 = (step0 + step) * kPrefKeys;
       int valid[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -478,7 +495,7 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
     // Softmax and PV of one step whose scores are st (may_mask false: the caller knows
     // the step needs no mask).
     auto finish = [&](int step, int stage, f32x16 st, const X8* vop, bool may_mask) {
-      const int kv0 = step * kPrefKeys;
+      const int kv0 = (step0 + step) * kPrefKeys;
       const bool masked = kv0 + kPrefKeys - 1 > qpos_min || kv0 + kPrefKeys > kv_end ||
                           ((badbits >> (2 * stage)) & 3u) != 0;
       if (may_mask && masked) {
@@ -567,12 +584,12 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
       // (The V reads may follow the upkeep: it writes no slot of this step.)
       u32x4 ka[KS];
       X8 vop[2 * DT];
-      if ((step + 1) * kPrefKeys <= qpos_last) {
+      if ((step0 + step + 1) * kPrefKeys <= qpos_last) {
         k_reads(nstage, ka);
         st_next = qk(ka);
       }
       if (mode != kNone) upkeep(step, stage, need, mode);
-      if (step * kPrefKeys <= qpos_last) {
+      if ((step0 + step) * kPrefKeys <= qpos_last) {
         v_reads(stage, vop);
         finish(step, stage, st_cur, vop, true);
       }
@@ -593,9 +610,10 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
     lds_barrier();
     {
       const int l = fresh_lane();
-      const int raw = l < a.max_tiles ? s_btw[l] : 0;
-      win_badm = __builtin_amdgcn_ballot_w64(l < a.max_tiles && (uint32_t)raw >= nb32);
-      btw = to_unit(raw, l);
+      const int w = (SPLIT ? win0 : 0) + l;
+      const int raw = w < a.max_tiles ? s_btw[l] : 0;
+      win_badm = __builtin_amdgcn_ballot_w64(w < a.max_tiles && (uint32_t)raw >= nb32);
+      btw = to_unit(raw, w);
     }
     stage_in(0, 0);
     if (nsteps > 1) stage_in(1, 1);
@@ -689,12 +707,13 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
     // wait while the ring is in full flow, staging of the steps that exist, clearing of
     // step + 2 (the last step can be partial).
     {
-      const int lim = (ctx + row0 + 1) / kPrefKeys - 1;   // t + 1 < steps below row0's first query
+      int lim = (ctx + row0 + 1) / kPrefKeys - 1 - step0;   // t + 1 < steps below row0's first query
+      if (SPLIT && lim > nsteps - 1) lim = nsteps - 1;      // t + 1 is one of the piece's steps
       // Issues step x into slot sl if it exists; the general path for a new table window,
       // a window with an invalid id, or a table row too short for the step.
       auto stage_fast = [&](int x, int sl) {
         if (x >= nsteps) return;
-        const int c0 = 2 * x;
+        const int c0 = 2 * (step0 + x);
         if (c0 >= win0 + 64 || win_badm || c0 + 1 >= a.max_tiles) {
           stage_in(x, sl);
           return;
@@ -718,8 +737,8 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
           const int wcols = win0 + 64 < a.max_tiles ? win0 + 64 : a.max_tiles;
           int end = lim;
           if (nsteps - NS + 1 < end) end = nsteps - NS + 1;            // step + NS - 1 exists
-          if (kv_end / kPrefKeys - 2 < end) end = kv_end / kPrefKeys - 2;   // step + 2 full
-          if ((wcols - 2 * NS + 2) / 2 < end) end = (wcols - 2 * NS + 2) / 2;  // columns
+          if (kv_end / kPrefKeys - 2 - step0 < end) end = kv_end / kPrefKeys - 2 - step0;   // step + 2 full
+          if ((wcols - 2 * NS + 2) / 2 - step0 < end) end = (wcols - 2 * NS + 2) / 2 - step0;  // columns
           for (; step < end; step += 2) {
             const int stage1 = stage + 1 == NS ? 0 : stage + 1;
             const int stage2 = stage1 + 1 == NS ? 0 : stage1 + 1;
@@ -733,7 +752,7 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
             {
               // This wave's tile of steps step + NS - 2 and step + NS - 1: tiles ci and
               // ci + 2 of the window.
-              const int ci = 2 * (step + NS - 2) + ld_blk - win0;
+              const int ci = 2 * (step0 + step + NS - 2) + ld_blk - win0;
               const uint32_t b0 = (uint32_t)__builtin_amdgcn_readlane(btw, ci);
               const uint32_t b1 = (uint32_t)__builtin_amdgcn_readlane(btw, ci + 2);
               const u16* base0 = (const u16*)((const char*)ld_head + (uint64_t)b0 * unit_bytes);
@@ -815,6 +834,21 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
 
     if (!wave_active) return;
     const float l = half_sum(l_run);
+    if constexpr (SPLIT) {
+      if (t.slot >= 0) {   // a piece of the tile: its partial, lane-major
+        const int64_t at = (int64_t)t.slot * kPrefWaves + wave;
+        const int ll = fresh_lane();
+        *reinterpret_cast<f32x2*>(a.ws_ml + (at * 64 + ll) * 2) = f32x2{m_run, l};
+        f32x4* const dst = reinterpret_cast<f32x4*>(a.ws_acc) + at * (4 * DT) * 64 + ll;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int b = 0; b < 4; ++b)
+            dst[(4 * dt + b) * 64] = f32x4{acc[dt][4 * b], acc[dt][4 * b + 1], acc[dt][4 * b + 2],
+                                           acc[dt][4 * b + 3]};
+        return;
+      }
+    }
     const float inv = l > 0.f ? 1.f / l : 0.f;
     // The output tile (32 rows x D, the size of one K or V plane of a stage) goes through
     // an LDS piece no wave reads after the tile's last barrier, so that every store
@@ -865,9 +899,91 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
     }
   };  // tile
 
+  const PrefTile none{-1, 0, 0, 0, 0, 0, 0, 0, -1};
+  if constexpr (SPLIT) {
+    // The tiles of a kv head end to end, each after kPrefPad empty slots; taker s of the kv
+    // head takes stream slots s C .. s C + C.  Every workgroup builds the same plan (the
+    // steps of each (sequence, query tile) and their prefix sum) in LDS.
+    __shared__ int32_t s_n[kPrefSplitTiles], s_at[kPrefSplitTiles];
+    __shared__ int32_t s_total;
+    const int NQ = a.num_qtiles, tiles = a.num_seqs * NQ;
+    for (int i = tid; i < tiles; i += blockDim.x) {
+      const int seq = i / NQ;
+      PrefTile pt = none;
+      pt.seq = seq;
+      pt.qtile = i - seq * NQ;
+      pt.tok0 = a.cu_seqlens[seq];
+      pt.tok1 = a.cu_seqlens[seq + 1];
+      pt.ctx = a.context_lens[seq];
+      int64_t tok0;
+      int n, ctx, steps = 0;
+      if (bounds(pt, tok0, n, ctx)) {
+        const int row_end = ((pt.qtile * kPrefWaves + kPrefWaves - 1) / a.group + 1) * kPrefRows;
+        steps = (ctx + (row_end < n ? row_end : n) + kPrefKeys - 1) / kPrefKeys;
+      }
+      s_n[i] = steps;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      int run = 0;
+      for (int base = 0; base < tiles; base += 64) {
+        const int i = base + lane;
+        const int n = i < tiles ? s_n[i] : 0;
+        const int v = n > 0 ? n + kPrefPad : 0;
+        int inc = v;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const int o = __shfl_up(inc, d, 64);
+          if (lane >= d) inc += o;
+        }
+        if (i < tiles) s_at[i] = run + inc - v + kPrefPad;   // its first step's slot
+        run += __builtin_amdgcn_readlane(inc, 63);
+      }
+      if (lane == 0) s_total = run;
+    }
+    __syncthreads();
+    const int total = __builtin_amdgcn_readfirstlane(s_total);
+    const int kvh = (int)(blockIdx.x % (unsigned)a.num_kv_heads);
+    const int taker = (int)(blockIdx.x / (unsigned)a.num_kv_heads);
+    int C = (total + a.takers - 1) / a.takers;
+    if (C < kPrefMinSteps) C = kPrefMinSteps;
+    if (blockIdx.x == 0) {   // the plan, for the merge
+      for (int i = tid; i < tiles; i += blockDim.x) a.ws_plan[2 + i] = s_n[i] > 0 ? s_at[i] : -1;
+      if (tid == 0) {
+        a.ws_plan[0] = C;
+        a.ws_plan[1] = tiles;
+      }
+    }
+    const int start = taker * C;
+    const int end = start + C < total ? start + C : total;
+    // the last tile whose first slot (its padding's) is at or before start
+    int i = 0;
+    for (int base = 0; base < tiles; base += 64) {
+      const int x = base + lane;
+      const uint64_t m = __builtin_amdgcn_ballot_w64(x < tiles && s_n[x] > 0 &&
+                                                     s_at[x] - kPrefPad <= start);
+      if (m == 0) continue;
+      i = base + 63 - __builtin_clzll(m);
+    }
+    for (; i < tiles; ++i) {
+      const int n = __builtin_amdgcn_readfirstlane(s_n[i]);
+      if (n == 0) continue;
+      const int at = __builtin_amdgcn_readfirstlane(s_at[i]);
+      if (at >= end) break;
+      const int b = start > at ? start - at : 0;
+      const int e = end - at < n ? end - at : n;
+      if (b >= e) continue;
+      PrefTile pt = look_up(i / NQ, i % NQ, kvh);
+      pt.sb = b;
+      pt.se = e;
+      if (b > 0 || e < n) pt.slot = 2 * (kvh * a.takers + taker) + (b > 0 ? 0 : 1);
+      tile(pt, none, [] {});
+    }
+    return;
+  }
+
   if (!a.persistent) {
-    tile(look_up(blockIdx.y, a.num_qtiles - 1 - (int)blockIdx.z, blockIdx.x),
-         PrefTile{-1, 0, 0, 0, 0, 0}, [] {});
+    tile(look_up(blockIdx.y, a.num_qtiles - 1 - (int)blockIdx.z, blockIdx.x), none, [] {});
     return;
   }
 
@@ -981,11 +1097,137 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
   }
 }
 
+template <int D, int NS, bool ROPE, bool F16>
+__global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(PrefillArgs a) {
+  prefill_body<D, NS, ROPE, F16, false>(a);
+}
+
+// The same tiles with their keys split over the workgroups: each takes the same number of
+// consecutive steps of its kv head's stream of tiles, and pieces of a tile leave partials
+// that prefill_merge_kernel adds.
+template <int D, int NS, bool ROPE, bool F16>
+__global__ __launch_bounds__(64 * kPrefWaves) void prefill_split_kernel(PrefillArgs a) {
+  prefill_body<D, NS, ROPE, F16, true>(a);
+}
+
+// One workgroup per (query tile, kv head, 32 columns of head_dim), wave w its job w: adds the tile's partials in
+// stream order, each scaled by 2^(m_p - M), in the accumulator's own lane layout.  Tiles
+// that one workgroup took whole were written by it.
+template <int D, bool F16>
+__global__ __launch_bounds__(64 * kPrefWaves) void prefill_merge_kernel(PrefillArgs a) {
+  using T = Elt<F16>;
+  constexpr int DT = D / 32;
+  const int i = blockIdx.x, kvh = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int C = a.ws_plan[0], at = a.ws_plan[2 + i];
+  if (at < 0) return;
+  const int seq = i / a.num_qtiles, qtile = i - seq * a.num_qtiles;
+  const int64_t tok0 = a.cu_seqlens[seq];
+  int64_t tok1 = a.cu_seqlens[seq + 1];
+  if (tok1 > a.num_tokens) tok1 = a.num_tokens;
+  const int n = (int)(tok1 - tok0);
+  const int ctx0 = a.context_lens[seq], ctx = ctx0 < 0 ? 0 : ctx0;
+  const int row_end = ((qtile * kPrefWaves + kPrefWaves - 1) / a.group + 1) * kPrefRows;
+  const int steps = (ctx + (row_end < n ? row_end : n) + kPrefKeys - 1) / kPrefKeys;
+  const int last = a.takers - 1;   // no context length leads past the takers' slots
+  const int s0 = min(at / C, last), s1 = min((at + steps - 1) / C, last);
+  if (s0 >= s1) return;
+  const int job = qtile * kPrefWaves + wave;
+  const int sub = job / a.group, head = kvh * a.group + job - sub * a.group;
+  const int row = sub * kPrefRows + (lane & 31), h = lane >> 5;
+  if (sub * kPrefRows >= n) return;   // a wave without rows
+  // Taker s holds its piece in slot 2 s of its kv head where it continues the tile, in
+  // 2 s + 1 where the tile begins with it (only s0).
+  auto slot = [&](int s) {
+    return ((int64_t)2 * (kvh * a.takers + s) + (s == s0 && s * C <= at ? 1 : 0)) * kPrefWaves +
+           wave;
+  };
+  float mx = kNegInf;
+  for (int s = s0; s <= s1; ++s) mx = fmaxf(mx, a.ws_ml[(slot(s) * 64 + lane) * 2]);
+  const int dt = blockIdx.z;   // 32 columns of head_dim per workgroup
+  f32x4 acc[4];
+#pragma unroll
+  for (int x = 0; x < 4; ++x) acc[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float l = 0.f;
+#pragma unroll 2
+  for (int s = s0; s <= s1; ++s) {
+    const int64_t p = slot(s);
+    const f32x2 ml = *reinterpret_cast<const f32x2*>(a.ws_ml + (p * 64 + lane) * 2);
+    const f32x4* const src =
+        reinterpret_cast<const f32x4*>(a.ws_acc) + (p * (4 * DT) + 4 * dt) * 64 + lane;
+    f32x4 v[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) v[x] = src[x * 64];
+    const float w = ml[0] == kNegInf ? 0.f : fast_exp2(ml[0] - mx);
+    l += ml[1] * w;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) acc[x] += v[x] * w;
+  }
+  if (row >= n) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  u16* const dst = a.out + ((tok0 + row) * a.num_heads + head) * (int64_t)D + 32 * dt + 4 * h;
+  // acc[b][e]: head_dim 32 dt + 8 b + 4 h + e of the lane's row
+#pragma unroll
+  for (int x = 0; x < 4; ++x)
+    *reinterpret_cast<u32x2*>(dst + 8 * x) = u32x2{T::pack(acc[x][0] * inv, acc[x][1] * inv),
+                                                   T::pack(acc[x][2] * inv, acc[x][3] * inv)};
+}
+
 }  // namespace ndl
 
 namespace ndl {
 
-// Shared by both entry points; cos == nullptr: q is already rotated.
+inline const void* prefill_split_fn(int head_dim, bool f16, bool rope) {
+  // [f16][head_dim 128][rope]
+  const void* const fns[2][2][2] = {
+      {{(const void*)prefill_split_kernel<64, 8, false, false>,
+        (const void*)prefill_split_kernel<64, 8, true, false>},
+       {(const void*)prefill_split_kernel<128, 6, false, false>,
+        (const void*)prefill_split_kernel<128, 6, true, false>}},
+      {{(const void*)prefill_split_kernel<64, 8, false, true>,
+        (const void*)prefill_split_kernel<64, 8, true, true>},
+       {(const void*)prefill_split_kernel<128, 6, false, true>,
+        (const void*)prefill_split_kernel<128, 6, true, true>}}};
+  return fns[f16 ? 1 : 0][head_dim == 128 ? 1 : 0][rope ? 1 : 0];
+}
+
+// The split launch's layout, or false where whole tiles are taken.  Whole tiles take as long
+// as the longest one, split ones the average over the GPU plus about 40 steps (a second ring
+// start per workgroup, the partials, the merge launch), so the split is taken where the
+// longest row's steps, times the share of the workgroups that the tiles leave idle, exceed
+// that.  us split / whole (graph of the launches): 32/8 heads of 128, 33 tokens after 4,000
+// 29.9 / 97.6 (118 steps saved), 500 after 4,000 59.9 / 108 (109); 14/2 of 64, 4 x 300 after
+// 2,000 36.7 / 48.2 (52), one prompt of 2,048 35.8 / 44.1 (36); 28/4 of 128, 4 x 300 after
+// 2,000 69.2 / 63.6 (31), 100 after 700 31.9 / 29.0 (23).  Once the tiles fill the GPU the
+// clock follows the matrix load and an even split gains nothing (8 x 400 after 4,000, 448
+// tiles: 259 / 236).
+constexpr int kPrefSplitGain = 40;
+struct PrefillSplit {
+  int64_t takers;
+  size_t plan_bytes, ml_bytes, bytes;
+};
+inline bool prefill_split(int num_seqs, int64_t num_tokens, int64_t qtiles, int num_heads,
+                          int num_kv_heads, int head_dim, int64_t max_tiles, PrefillSplit* sp) {
+  const int64_t tiles = num_seqs * qtiles;   // of the plan: an upper bound per kv head
+  if (tiles > kPrefSplitTiles || max_tiles * 16 < NDL_PREFILL_SPLIT_MIN_KEYS ||
+      max_tiles > (1 << 20))
+    return false;
+  int64_t slots = resident_workgroups(prefill_split_fn(head_dim, false, true), 64 * kPrefWaves);
+  if (slots <= 0) slots = 256;
+  sp->takers = slots / num_kv_heads;
+  if (sp->takers < 2) return false;
+  // workgroups whole tiles would keep busy: eight 32-row jobs each
+  const int64_t busy = (num_tokens / kPrefRows + num_seqs) * num_heads / kPrefWaves;
+  if (busy >= slots || max_tiles / 2 * (slots - busy) < kPrefSplitGain * slots) return false;
+  const size_t n = (size_t)2 * sp->takers * num_kv_heads * kPrefWaves * 64;   // lanes
+  sp->plan_bytes = ((2 + (size_t)tiles) * sizeof(int32_t) + 255) & ~(size_t)255;
+  sp->ml_bytes = n * 2 * sizeof(float);
+  sp->bytes = sp->plan_bytes + sp->ml_bytes + n * (head_dim / 2) * sizeof(float);
+  return true;
+}
+
+// Shared by the entry points; cos == nullptr: q is already rotated.  A workspace lets the
+// launch split its tiles' keys (prefill_split).
 static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const void* cos,
                           const void* sin, int64_t cs_tok_stride, const void* kv_cache,
                           int64_t num_blocks, const int32_t* block_table, int64_t bt_row_stride,
@@ -993,7 +1235,8 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
                           const int32_t* context_lens, int num_seqs, int64_t num_tokens,
                           int max_seqlen, int max_context_len, int num_heads, int num_kv_heads,
                           int head_dim, int block_size, int dtype, float scale,
-                          ndl_stream_t stream) {
+                          ndl_stream_t stream, void* workspace = nullptr,
+                          size_t workspace_bytes = 0) {
   if (!dtype_known(dtype)) return NDL_ERR_UNSUPPORTED;
   const int tshift = block_tile_shift(block_size);
   if (tshift < 0 || (head_dim != 64 && head_dim != 128)) return NDL_ERR_UNSUPPORTED;
@@ -1060,6 +1303,37 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
   a.num_seqs = num_seqs;
   a.persistent = num_seqs <= kPrefListSeqs && qtiles <= kPrefListLevels &&
                  gx * (int64_t)num_seqs * qtiles < ((int64_t)1 << 31);
+  const bool f16 = dtype_is_f16(dtype);
+  PrefillSplit sp;
+  if (workspace != nullptr && ((uintptr_t)workspace & 15u) == 0 &&
+      prefill_split(num_seqs, num_tokens, qtiles, num_heads, num_kv_heads, head_dim, a.max_tiles,
+                    &sp) &&
+      workspace_bytes >= sp.bytes) {
+    a.takers = (int)sp.takers;
+    a.ws_plan = (int32_t*)workspace;
+    a.ws_ml = (float*)((char*)workspace + sp.plan_bytes);
+    a.ws_acc = (float*)((char*)workspace + sp.plan_bytes + sp.ml_bytes);
+    const void* const fn = prefill_split_fn(head_dim, f16, rope);
+    void* args[] = {&a};
+    if (hipLaunchKernel(fn, dim3((unsigned)(sp.takers * gx)), dim3(64 * waves), args, 0, s) !=
+        hipSuccess) {
+      (void)hipGetLastError();
+      return NDL_ERR_LAUNCH;
+    }
+    const int rc = check_launch();
+    if (rc != NDL_OK) return rc;
+    const void* const mfn =
+        head_dim == 128 ? (f16 ? (const void*)prefill_merge_kernel<128, true>
+                               : (const void*)prefill_merge_kernel<128, false>)
+                        : (f16 ? (const void*)prefill_merge_kernel<64, true>
+                               : (const void*)prefill_merge_kernel<64, false>);
+    if (hipLaunchKernel(mfn, dim3((unsigned)(num_seqs * qtiles), (unsigned)gx, head_dim / 32),
+                        dim3(64 * waves), args, 0, s) != hipSuccess) {
+      (void)hipGetLastError();
+      return NDL_ERR_LAUNCH;
+    }
+    return check_launch();
+  }
   // [f16][head_dim 128][rope]
   const void* const fns[2][2][2] = {
       {{(const void*)varlen_prefill_kernel<64, 8, false, false>,
@@ -1070,7 +1344,7 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
         (const void*)varlen_prefill_kernel<64, 8, true, true>},
        {(const void*)varlen_prefill_kernel<128, 6, false, true>,
         (const void*)varlen_prefill_kernel<128, 6, true, true>}}};
-  const void* fn = fns[dtype_is_f16(dtype) ? 1 : 0][head_dim == 128 ? 1 : 0][rope ? 1 : 0];
+  const void* fn = fns[f16 ? 1 : 0][head_dim == 128 ? 1 : 0][rope ? 1 : 0];
   dim3 grid((unsigned)gx, (unsigned)num_seqs, (unsigned)qtiles);
   if (a.persistent) {
     const int64_t slots = resident_workgroups(fn, 64 * waves);
@@ -1119,4 +1393,40 @@ extern "C" int ndl_rope_varlen_prefill(void* out, const void* q, int64_t q_tok_s
                              cu_seqlens, context_lens, num_seqs, num_tokens, max_seqlen,
                              max_context_len, num_heads, num_kv_heads, head_dim, block_size,
                              dtype, scale, stream);
+}
+
+extern "C" size_t ndl_varlen_prefill_workspace_bytes(int num_seqs, int64_t num_tokens,
+                                                     int max_seqlen, int max_blocks_per_seq,
+                                                     int num_heads, int num_kv_heads,
+                                                     int head_dim, int block_size, int dtype) {
+  using namespace ndl;
+  const int tshift = block_tile_shift(block_size);
+  if (!dtype_supported(dtype) || tshift < 0 || (head_dim != 64 && head_dim != 128) ||
+      num_seqs <= 0 || num_tokens <= 0 || max_seqlen <= 0 || max_blocks_per_seq <= 0 ||
+      num_kv_heads <= 0 || num_heads <= 0 || num_heads % num_kv_heads != 0)
+    return 0;
+  const int64_t qtiles = (((int64_t)max_seqlen + kPrefRows - 1) / kPrefRows *
+                              (num_heads / num_kv_heads) + kPrefWaves - 1) / kPrefWaves;
+  PrefillSplit sp;
+  return prefill_split(num_seqs, num_tokens, qtiles, num_heads, num_kv_heads, head_dim,
+                       (int64_t)max_blocks_per_seq << tshift, &sp)
+             ? sp.bytes
+             : 0;
+}
+
+extern "C" int ndl_varlen_prefill_split(void* out, const void* q, int64_t q_tok_stride,
+                                        const void* cos, const void* sin, int64_t cs_tok_stride,
+                                        const void* kv_cache, int64_t num_blocks,
+                                        const int32_t* block_table, int64_t bt_row_stride,
+                                        int max_blocks_per_seq, const int32_t* cu_seqlens,
+                                        const int32_t* context_lens, int num_seqs,
+                                        int64_t num_tokens, int max_seqlen, int max_context_len,
+                                        int num_heads, int num_kv_heads, int head_dim,
+                                        int block_size, int dtype, float scale, void* workspace,
+                                        size_t workspace_bytes, ndl_stream_t stream) {
+  return ndl::launch_prefill(out, q, q_tok_stride, cos, sin, cs_tok_stride, kv_cache,
+                             num_blocks, block_table, bt_row_stride, max_blocks_per_seq,
+                             cu_seqlens, context_lens, num_seqs, num_tokens, max_seqlen,
+                             max_context_len, num_heads, num_kv_heads, head_dim, block_size,
+                             dtype, scale, stream, workspace, workspace_bytes);
 }

@@ -402,11 +402,24 @@ def varlen_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.T
     if _validate_enabled():
         _validate_slots(block_table, num_blocks)
     lib = _lib.load()
-    tail = (kv_cache.data_ptr(), num_blocks,
+    args = (kv_cache.data_ptr(), num_blocks,
             block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
             cu_seqlens.data_ptr(), context_lens.data_ptr(), n_seqs, n_tok, int(max_seqlen),
             int(max_context_len), num_heads, num_kv_heads, head_dim, bs, _DTYPES[q.dtype],
-            float(scale), _stream(dev))
+            float(scale))
+    # few query tiles over many keys: split over workgroups, the pieces in a workspace
+    need = 0
+    if block_table.shape[1] * bs >= _lib.NDL_PREFILL_SPLIT_MIN_KEYS:
+        need = lib.ndl_varlen_prefill_workspace_bytes(
+            n_seqs, n_tok, int(max_seqlen), block_table.shape[1], num_heads, num_kv_heads,
+            head_dim, bs, _DTYPES[q.dtype])
+    if need:
+        ws = torch.empty(need, dtype=torch.uint8, device=dev)
+        rc = lib.ndl_varlen_prefill_split(out.data_ptr(), q.data_ptr(), qs, _ptr(cos), _ptr(sin),
+                                          cs, *args, ws.data_ptr(), need, _stream(dev))
+        _lib.check(rc, "ndl_varlen_prefill_split")
+        return out
+    tail = (*args, _stream(dev))
     if cos is None:
         rc = lib.ndl_varlen_prefill(out.data_ptr(), q.data_ptr(), qs, *tail)
         _lib.check(rc, "ndl_varlen_prefill")
