@@ -6,9 +6,13 @@
 // in fp32.  As ndl_varlen_prefill does for the 16-bit formats, K/V are read back through
 // block_table after the append (attention.py:103), which also covers a cached prefix.
 //
-// One wave per (query head, 16 query rows); four waves per workgroup take consecutive row
-// blocks of one head.  The tile math is the float32 decode's (paged_decode_f32.hip) with the
-// N dimension holding the 16 query rows of one head instead of the heads of one token:
+// Four waves per workgroup take 16 or 32 consecutive rows of one query head, sharing the keys
+// of each 16-row block (every fourth or second 16-key tile a wave, combined through LDS at
+// the end); the row blocks with the most keys are dispatched first.  The bound is the fp32
+// matrix rate (1,024 or 2,048 cycles per tile and SIMD at head_dim 64 or 128) and, once the
+// GPU is full, the L2: without LDS sharing a wave reads 8 or 16 KB per tile.  The tile math is
+// the float32 decode's (paged_decode_f32.hip) with the N dimension holding the 16 query rows
+// of one head instead of the heads of one token:
 //   * S^T = K q^T on v_mfma_f32_16x16x4_f32: lane (i, kk) = (lane % 16, lane / 16) holds
 //     K[key i][16 m + 4 kk + e] and q[row i][16 m + 4 kk + e];
 //   * the accumulator holds keys 4 kk + r of row i in lane (i, kk), the B operand of
@@ -23,9 +27,6 @@
 #include "ndl_common.hpp"
 
 namespace ndl {
-
-constexpr int kPrefF32Waves = 4;
-constexpr int kPrefF32Rows = 16 * kPrefF32Waves;   // query rows per workgroup
 
 struct PrefillF32Args {
   float* out;
@@ -48,19 +49,27 @@ struct PrefillF32Args {
   const float* rope_cos;   // null: q is already rotated
   const float* rope_sin;
   int64_t rope_stride;
+  int last_block;   // the row block of blockIdx.z = 0; later ones take earlier rows
 };
 
 __device__ __forceinline__ f32x4 ldf4p(const float* p) {
   return *reinterpret_cast<const f32x4*>(p);
 }
 
-template <int D, bool ROPE>
-__global__ __launch_bounds__(64 * kPrefF32Waves) void varlen_prefill_f32_kernel(PrefillF32Args a) {
+// Two waves per SIMD at head_dim 128: left to itself the compiler takes accumulation registers
+// past the 256 that allow it (16 prompts of 400 tokens, 28/4 heads: 369 us against 286).
+template <int D, bool ROPE, int NWK, int NWR>
+__global__ __launch_bounds__(64 * NWK * NWR) __attribute__((amdgpu_waves_per_eu(
+    D == 128 ? 2 : 1))) void varlen_prefill_f32_kernel(PrefillF32Args a) {
+  constexpr int NW = NWK * NWR;
   constexpr int QK = D / 16;
   constexpr int G = D / 64;
+  constexpr int E = D / 4;     // accumulator floats per lane
+  constexpr int KPW = E / NWK; // of which each wave finishes
   static_assert(D == 64 || D == 128, "head_dim");
   const int head = blockIdx.x, seq = blockIdx.y;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int i16 = lane & 15, kk = lane >> 4;
   const int kvh = head / a.group;
 
@@ -69,23 +78,26 @@ __global__ __launch_bounds__(64 * kPrefF32Waves) void varlen_prefill_f32_kernel(
   if (tok1 > a.num_tokens) tok1 = a.num_tokens;
   if (tok0 < 0 || tok1 <= tok0) return;
   const int n = (int)(tok1 - tok0);
-  const int r0 = (int)blockIdx.z * kPrefF32Rows + 16 * wv;   // this wave's first row
-  if (r0 >= n) return;   // no barriers in this kernel
+  // the workgroup's first row: the blocks with the most keys are dispatched first
+  const int wk = wv % NWK, wr = wv / NWK;   // the wave's share of the keys, its rows
+  const int wg_r0 = (a.last_block - (int)blockIdx.z) * 16 * NWR;
+  if (wg_r0 >= n) return;
+  const int r0 = wg_r0 + 16 * wr;   // the wave's first row
   const int ctx0 = a.context_lens[seq];
   const int ctx = ctx0 < 0 ? 0 : ctx0;
-  const int row = r0 + i16;                       // this lane's query row
-  const bool row_ok = row < n;
-  const int64_t qpos = (int64_t)ctx + row;        // its position in the sequence
-  const int64_t kv_end = (int64_t)ctx + (r0 + 16 < n ? r0 + 16 : n);   // keys the wave reads
-  const int ntk = (int)((kv_end + 15) >> 4);      // 16-key tiles
+  const int64_t kv_end = (int64_t)ctx + (r0 + 16 < n ? r0 + 16 : n);   // keys read
+  const int ntk = r0 < n ? (int)((kv_end + 15) >> 4) : 0;      // 16-key tiles
+  const int ntw = wk < ntk ? (ntk - wk + NWK - 1) / NWK : 0;   // this wave's: wk, wk + NWK, ..
   const int tshift = a.tile_shift, tmask = (1 << tshift) - 1;
   const int64_t blk_stride = (int64_t)a.num_kv_heads * (16 << tshift) * D;
   const int64_t head_off = (int64_t)kvh * (16 << tshift) * D;
 
-  // q^T operand of the lane's row (a row past the range reads the wave's first row)
+  // q^T operand of the lane's row (a row past the range reads the workgroup's first row)
+  const int row = r0 + i16;
+  const int64_t qpos = (int64_t)ctx + row;        // its position in the sequence
   f32x4 qv[QK];
   {
-    const int64_t t = tok0 + (row_ok ? row : r0);
+    const int64_t t = tok0 + (row < n ? row : wg_r0);
     const float* qrow = a.q + t * a.q_tok_stride + (int64_t)head * D + 4 * kk;
 #pragma unroll
     for (int m = 0; m < QK; ++m) qv[m] = ldf4p(qrow + 16 * m);
@@ -120,9 +132,9 @@ __global__ __launch_bounds__(64 * kPrefF32Waves) void varlen_prefill_f32_kernel(
   const int32_t* bt_row = a.block_table + (int64_t)seq * a.bt_row_stride;
   const int max_tiles = a.max_blocks << tshift;
 
-  for (int w0 = 0; w0 < ntk; w0 += 64) {
-    const int cnt = ntk - w0 < 64 ? ntk - w0 : 64;
-    int tl = w0 + (lane < cnt ? lane : cnt - 1);
+  for (int w0 = 0; w0 < ntw; w0 += 64) {
+    const int cnt = ntw - w0 < 64 ? ntw - w0 : 64;
+    int tl = wk + NWK * (w0 + (lane < cnt ? lane : cnt - 1));
     if (tl > max_tiles - 1) tl = max_tiles - 1;   // the table row's clamp
     const int bt_lane = bt_row[tl >> tshift];
     asm volatile("" ::"v"(bt_lane));   // the ids are waited for once per window
@@ -131,7 +143,7 @@ __global__ __launch_bounds__(64 * kPrefF32Waves) void varlen_prefill_f32_kernel(
     auto load_tile = [&](int it, Tile& t, bool live) {
       const int itc = it < cnt ? it : cnt - 1;
       int64_t blk = __builtin_amdgcn_readlane(bt_lane, itc);
-      int tix = w0 + itc;
+      int tix = wk + NWK * (w0 + itc);
       if (tix > max_tiles - 1) tix = max_tiles - 1;
       t.bad = blk < 0 || blk >= a.num_blocks;
       if (t.bad) blk = 0;
@@ -146,26 +158,33 @@ __global__ __launch_bounds__(64 * kPrefF32Waves) void varlen_prefill_f32_kernel(
         for (int t4 = 0; t4 < 4; ++t4) t.v[g][t4] = ldf4p(vb + (live ? t4 * D + 64 * g : 0));
     };
     auto compute = [&](int it, Tile& t) {
-      const int64_t key0 = (int64_t)(w0 + it) * 16 + 4 * kk;
+      const int64_t tile0 = (int64_t)(wk + NWK * (w0 + it)) * 16;   // the tile's first key
+      const int64_t key0 = tile0 + 4 * kk;
       f32x4 st = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int m = 0; m < QK; ++m)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           st = __builtin_amdgcn_mfma_f32_16x16x4f32(t.k[m][e], qv[m][e], st, 0, 0, 0);
-      // st[r]: key key0 + r for the lane's row
-      float sc[4];
+      // st[r]: key key0 + r for the lane's row.  Tiles that end at or before the first row's
+      // position need no mask (wave-uniform).
+      if (t.bad || tile0 + 16 > (int64_t)ctx + r0 + 1) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int64_t key = key0 + r;
+          const bool in_range = !t.bad && key < kv_end;
+          st[r] = in_range && key <= qpos ? st[r] : kNegInf;
+          if (!in_range) {   // rows that may hold any bits (NaN * 0 = NaN): cleared
+#pragma unroll
+            for (int g = 0; g < G; ++g) t.v[g][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+        }
+      }
       float mt = kNegInf;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int64_t key = key0 + r;
-        const bool in_range = !t.bad && key < kv_end;
-        sc[r] = in_range && key <= qpos ? st[r] * a.scale_log2 : kNegInf;
-        mt = fmaxf(mt, sc[r]);
-        if (!in_range) {   // rows that may hold any bits (NaN * 0 = NaN): cleared
-#pragma unroll
-          for (int g = 0; g < G; ++g) t.v[g][r] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+        st[r] *= a.scale_log2;
+        mt = fmaxf(mt, st[r]);
       }
       mt = max_xor32(max_xor16(mt));
       const float m_new = fmaxf(m_run, mt);
@@ -175,7 +194,7 @@ __global__ __launch_bounds__(64 * kPrefF32Waves) void varlen_prefill_f32_kernel(
       float ps = 0.f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        p[r] = fast_exp2(sc[r] - m_use);
+        p[r] = fast_exp2(st[r] - m_use);
         ps += p[r];
       }
       l_run = l_run * alpha + ps;
@@ -187,13 +206,13 @@ __global__ __launch_bounds__(64 * kPrefF32Waves) void varlen_prefill_f32_kernel(
           for (int e = 0; e < 4; ++e) acc[g][e] *= alpha;
       }
 #pragma unroll
-      for (int g = 0; g < G; ++g)
+      for (int t4 = 0; t4 < 4; ++t4)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+        for (int g = 0; g < G; ++g)
 #pragma unroll
-          for (int t4 = 0; t4 < 4; ++t4)
-            acc[g][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(t.v[g][t4][e], p[t4], acc[g][e],
-                                                             0, 0, 0);
+          for (int e = 0; e < 4; ++e)
+            acc[g][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(t.v[g][t4][e], p[t4], acc[g][e], 0,
+                                                             0, 0);
     };
     Tile buf[2];
     load_tile(0, buf[0], true);
@@ -204,16 +223,73 @@ __global__ __launch_bounds__(64 * kPrefF32Waves) void varlen_prefill_f32_kernel(
       if (it + 1 < cnt) compute(it + 1, buf[1]);
     }
   }
+
   l_run = add_xor32(add_xor16(l_run));
-  if (!row_ok) return;
-  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-  float* const dst = a.out + ((tok0 + row) * a.num_heads + head) * (int64_t)D + 16 * kk;
+
+  // Combine over the waves of the same rows, as the float32 decode does: m, l and accumulators
+  // into LDS, one barrier, then wave (wk, wr) sums elements wk * KPW .. of every lane over the
+  // NWK waves in a fixed order.  Lane element x = (4 g + r) * 4 + e holds
+  // O[row i16][64 g + 16 kk + 4 r + e].
+  __shared__ __attribute__((aligned(16))) float sacc[NW * E * 64];
+  __shared__ float sm[NW * 16], sl[NW * 16];
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      *reinterpret_cast<f32x4*>(dst + 64 * g + 4 * r) =
-          f32x4{acc[g][0][r] * inv, acc[g][1][r] * inv, acc[g][2][r] * inv, acc[g][3][r] * inv};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sacc[(wv * E + (4 * g + r) * 4 + e) * 64 + lane] = acc[g][e][r];
+  if (kk == 0) {
+    sm[wv * 16 + i16] = m_run;
+    sl[wv * 16 + i16] = l_run;
+  }
+  __syncthreads();
+  if (row >= n) return;
+  const int w0 = wr * NWK;   // the waves of these rows
+  float mw[NWK];
+  float mx = kNegInf;
+#pragma unroll
+  for (int w = 0; w < NWK; ++w) {
+    mw[w] = sm[(w0 + w) * 16 + i16];
+    mx = fmaxf(mx, mw[w]);
+  }
+  float den = 0.f, o[KPW];
+#pragma unroll
+  for (int x = 0; x < KPW; ++x) o[x] = 0.f;
+#pragma unroll
+  for (int w = 0; w < NWK; ++w) {
+    const float wt = mw[w] == kNegInf ? 0.f : fast_exp2(mw[w] - mx);
+    den += __fmul_rn(sl[(w0 + w) * 16 + i16], wt);
+#pragma unroll
+    for (int x = 0; x < KPW; ++x)
+      o[x] += __fmul_rn(sacc[((w0 + w) * E + wk * KPW + x) * 64 + lane], wt);
+  }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  float* const orow = a.out + ((tok0 + row) * a.num_heads + head) * (int64_t)D + 16 * kk;
+  static_assert(KPW % 4 == 0, "whole 16-byte pieces per wave");
+#pragma unroll
+  for (int x = 0; x < KPW; x += 4) {   // consecutive e of (g, r) = (x / 16, x / 4 % 4)
+    const int x0 = wk * KPW + x;
+    *reinterpret_cast<f32x4*>(orow + 64 * (x0 / 16) + 4 * ((x0 / 4) % 4)) =
+        f32x4{o[x] * inv, o[x + 1] * inv, o[x + 2] * inv, o[x + 3] * inv};
+  }
+}
+
+// The split of a workgroup's four waves.  Four over the keys of 16 rows keep the longest row
+// block's chain short, and a small batch's time is that chain; two over the keys of 32 rows
+// read each K/V tile half as often, which a batch that fills the GPU is bound by.  us at
+// 4 x 1 / 2 x 2 (1 x 4, the split before, in brackets): 14/2 heads of 64, prompts of 64 to
+// 1,024 tokens, 2,168 in all, 49.5 / 69 (110); 28/4 of 128, 33 tokens after 2,000 54 / 94
+// (175), 1,000 118 / 121 (110), 6 x 500 199 / 176 (180), 8 x 1,000 979 / 757 (738), 16 x 400
+// 376 / 286 (346).  The line: row blocks of 16, scaled by how even the prompts are (a batch
+// of uneven ones is as long as its longest), against 1.5 per SIMD.
+constexpr double kPrefF32Blocks = 1536;
+
+template <int NWK, int NWR>
+const void* prefill_f32_fn(int head_dim, bool rope) {
+  return head_dim == 128 ? (rope ? (const void*)varlen_prefill_f32_kernel<128, true, NWK, NWR>
+                                 : (const void*)varlen_prefill_f32_kernel<128, false, NWK, NWR>)
+                         : (rope ? (const void*)varlen_prefill_f32_kernel<64, true, NWK, NWR>
+                                 : (const void*)varlen_prefill_f32_kernel<64, false, NWK, NWR>);
 }
 
 int launch_prefill_f32(void* out, const void* q, int64_t q_tok_stride, const void* cos,
@@ -225,8 +301,12 @@ int launch_prefill_f32(void* out, const void* q, int64_t q_tok_stride, const voi
                        int head_dim, int block_size, float scale, ndl_stream_t stream) {
   (void)max_context_len;
   if ((q_tok_stride & 3) || (cos != nullptr && (cs_tok_stride & 3))) return NDL_ERR_INVALID_ARG;
-  const int64_t zb = ((int64_t)max_seqlen + kPrefF32Rows - 1) / kPrefF32Rows;
-  if (num_seqs > 65535 || zb > 65535) return NDL_ERR_UNSUPPORTED;
+  const double even = (double)num_tokens / ((double)num_seqs * max_seqlen);
+  const double blocks = ((double)num_tokens / 16 + num_seqs) * num_heads;
+  const bool wide = blocks * (even < 1 ? even : 1) >= kPrefF32Blocks;
+  const int rows = wide ? 32 : 16;   // per workgroup
+  const int64_t zb = ((int64_t)max_seqlen + rows - 1) / rows;
+  if (num_seqs > 65535 || ((int64_t)max_seqlen + 63) / 64 > 65535) return NDL_ERR_UNSUPPORTED;
   PrefillF32Args a;
   a.out = (float*)out;
   a.q = (const float*)q;
@@ -249,18 +329,21 @@ int launch_prefill_f32(void* out, const void* q, int64_t q_tok_stride, const voi
   a.rope_sin = (const float*)sin;
   a.rope_stride = cs_tok_stride;
   const bool rope = cos != nullptr;
-  const void* fn = head_dim == 128
-      ? (rope ? (const void*)varlen_prefill_f32_kernel<128, true>
-              : (const void*)varlen_prefill_f32_kernel<128, false>)
-      : (rope ? (const void*)varlen_prefill_f32_kernel<64, true>
-              : (const void*)varlen_prefill_f32_kernel<64, false>);
+  const void* fn = wide ? prefill_f32_fn<2, 2>(head_dim, rope) : prefill_f32_fn<4, 1>(head_dim, rope);
   void* args[] = {&a};
-  if (hipLaunchKernel(fn, dim3((unsigned)num_heads, (unsigned)num_seqs, (unsigned)zb),
-                      dim3(64 * kPrefF32Waves), args, 0, (hipStream_t)stream) != hipSuccess) {
-    (void)hipGetLastError();
-    return NDL_ERR_LAUNCH;
+  constexpr int64_t kMaxZ = 65535;   // a grid's z dimension
+  for (int64_t z = 0; z < zb; z += kMaxZ) {
+    a.last_block = (int)(zb - 1 - z);
+    const int64_t nz = zb - z < kMaxZ ? zb - z : kMaxZ;
+    if (hipLaunchKernel(fn, dim3((unsigned)num_heads, (unsigned)num_seqs, (unsigned)nz),
+                        dim3(256), args, 0, (hipStream_t)stream) != hipSuccess) {
+      (void)hipGetLastError();
+      return NDL_ERR_LAUNCH;
+    }
+    const int rc = check_launch();
+    if (rc != NDL_OK) return rc;
   }
-  return check_launch();
+  return NDL_OK;
 }
 
 }  // namespace ndl
