@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 from pathlib import Path
 
 import torch  # noqa: F401  (loads torch's HIP runtime before ours)
@@ -180,6 +181,9 @@ _SIGNATURES = {
 }
 
 _LIB = None
+# The native bindings (csrc/bind.cpp) over the loaded library, or None: ops.py runs its own
+# path then, with the same results.
+NATIVE = None
 
 
 class NeedleAmdError(RuntimeError):
@@ -205,7 +209,22 @@ def load() -> ctypes.CDLL:
     if ver != NDL_ABI_VERSION:
         raise NeedleAmdError(f"ABI version {ver} != expected {NDL_ABI_VERSION}")
     _LIB = lib
+    _load_native(lib)
     return lib
+
+
+def _load_native(lib: ctypes.CDLL) -> None:
+    global NATIVE
+    try:
+        from . import _native
+    except ImportError as e:
+        warnings.warn(f"needle_amd._native not usable ({e}): build it with `make -C "
+                      "needle_amd/csrc`; eager launches go through the interpreter until then")
+        NATIVE = None
+        return
+    _native.init({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+                  for name in EXPORTED_SYMBOLS})
+    NATIVE = _native
 
 
 def check(status: int, what: str) -> None:

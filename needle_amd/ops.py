@@ -147,6 +147,10 @@ def rope_kv_append(q: Optional[torch.Tensor], k: torch.Tensor, v: torch.Tensor,
     q=None rotates and appends k (and appends v) only, and returns None: the form that
     precedes rope_varlen_prefill, which rotates q itself.
     """
+    if q is None and out is None and cu_seqlens is not None and _lib.NATIVE is not None:
+        if _lib.NATIVE.rope_kv_append(k, v, cos, sin, kv_cache, block_table, context_lens,
+                                      cu_seqlens):
+            return None
     _check_cache(kv_cache)
     dev = kv_cache.device
     _, num_blocks, hkv, bs, d = kv_cache.shape
@@ -364,6 +368,12 @@ def varlen_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.T
     rope_kv_append's rotated q fed to this function, with k already rotated in the cache
     (rope_kv_append with q=None).
     """
+    if out is None and _lib.NATIVE is not None:
+        out = _lib.NATIVE.varlen_prefill(q, kv_cache, block_table, cu_seqlens, context_lens,
+                                         max_seqlen, scale, num_heads, num_kv_heads, head_dim,
+                                         max_context_len, cos, sin)
+        if out is not None:
+            return out
     _check_cache(kv_cache)
     dev = kv_cache.device
     _, num_blocks, hkv, bs, d = kv_cache.shape
@@ -509,6 +519,10 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     x: [rows, hidden] with contiguous rows; residual: [rows, hidden]; weight: [hidden];
     one dtype (bfloat16, float16 or float32), on one GPU.
     """
+    if _lib.NATIVE is not None:
+        done = _lib.NATIVE.rms_norm(x, weight, eps, residual)
+        if done is not None:
+            return done
     _require(x.is_cuda, "x must be a GPU tensor")
     if x.dtype not in _DTYPES:
         raise TypeError(f"unsupported dtype {x.dtype}")
@@ -539,6 +553,10 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     torch's roundings (the SiLU rounded to the dtype, then the product).  gate, up:
     [rows, intermediate] with contiguous rows (e.g. the two halves of one fused gate/up
     projection output); returns a new [rows, intermediate] tensor."""
+    if _lib.NATIVE is not None:
+        done = _lib.NATIVE.silu_mul(gate, up)
+        if done is not None:
+            return done
     _require(gate.is_cuda, "gate must be a GPU tensor")
     if gate.dtype not in _DTYPES:
         raise TypeError(f"unsupported dtype {gate.dtype}")
