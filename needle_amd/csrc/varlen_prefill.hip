@@ -1299,7 +1299,7 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
 
   hipStream_t s = (hipStream_t)stream;
   // Persistent launch (one resident workgroup per slot, walking the longest-first tile
-  // list) unless the list would not fit in LDS.
+  // list) unless the list would not fit in LDS or every tile has a slot of its own.
   a.num_seqs = num_seqs;
   a.persistent = num_seqs <= kPrefListSeqs && qtiles <= kPrefListLevels &&
                  gx * (int64_t)num_seqs * qtiles < ((int64_t)1 << 31);
@@ -1349,8 +1349,13 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
   if (a.persistent) {
     const int64_t slots = resident_workgroups(fn, 64 * waves);
     if (slots <= 0) return NDL_ERR_LAUNCH;
-    const int64_t items = gx * (int64_t)num_seqs * qtiles;   // upper bound of the list
-    grid = dim3((unsigned)(items < slots ? items : slots), 1, 1);
+    // With a slot for every tile (an upper bound of them) each is its own workgroup: nothing to
+    // balance, and the list's build is saved (one prompt of 77 tokens, with its append, 12.7 ->
+    // 10.3 us).
+    if (gx * (int64_t)num_seqs * qtiles <= slots)
+      a.persistent = 0;
+    else
+      grid = dim3((unsigned)slots, 1, 1);
   }
   void* args[] = {&a};
   if (hipLaunchKernel(fn, grid, dim3(64 * waves), args, 0, s) != hipSuccess) {
