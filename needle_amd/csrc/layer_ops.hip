@@ -17,7 +17,7 @@
 // of the sum of squares differs from torch's reduction, which can move the statistic by an
 // ulp and an element of the output by an ulp of its format now and then.
 //
-// Both kernels are latency-bound at decode sizes (one row per wave, tens of rows) and
+// Both kernels are latency-bound at decode sizes (tens of rows) and
 // HBM-bound at prefill sizes: every element is read and written once.
 #include "ndl_common.hpp"
 
@@ -25,7 +25,7 @@ namespace ndl {
 namespace {
 
 constexpr int kThreads = 256;           // four waves
-constexpr int kMaxHidden = 8192;        // 16 chunks of 8 elements per lane
+constexpr int kMaxHidden = 8192;        // four chunks of 8 elements per lane of four waves
 
 // Eight consecutive elements of a row as fp32 (16 bytes of a 16-bit format, 32 of float32).
 template <int FMT>
@@ -91,46 +91,104 @@ struct NormArgs {
   float eps, inv_hidden;
 };
 
-// One wave per row; lane l holds chunks l, l + 64, .. (8 elements each) of the row, and the
-// same chunks of the weight (loaded with the row: one memory round trip), in registers
-// between the statistic and the products.
-template <int FMT, int NC, bool RES>
+// Eight elements as loaded.
+template <int FMT>
+struct Raw8 {
+  u32x4 v[FMT == kFmtF32 ? 2 : 1];
+};
+template <int FMT>
+__device__ __forceinline__ Raw8<FMT> raw8(const void* p) {
+  Raw8<FMT> r;
+  r.v[0] = ld16(p);
+  if constexpr (FMT == kFmtF32) r.v[1] = ld16(static_cast<const char*>(p) + 16);
+  return r;
+}
+template <int FMT>
+__device__ __forceinline__ void unpack8(const Raw8<FMT>& r, float (&v)[8]) {
+  if constexpr (FMT == kFmtF32) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = __uint_as_float(r.v[0][i]);
+      v[4 + i] = __uint_as_float(r.v[1][i]);
+    }
+  } else {
+    using T = Elt<FMT == kFmtF16>;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = T::lo(r.v[0][i]);
+      v[2 * i + 1] = T::hi(r.v[0][i]);
+    }
+  }
+}
+
+// WPR waves per row; lane l of wave w holds chunks 64 w + l, + 64 WPR, .. (8 elements each) of
+// the row, and the same chunks of the weight, in registers between the statistic and the
+// products.  Every load goes out before any store (the compiler cannot move a load over the
+// store of the residual sum, which may be the residual's own memory), and lanes past the row
+// load its last chunk again instead of branching, so a row costs one memory round trip:
+// interleaved with the stores it cost one per chunk.
+template <int FMT, int NC, bool RES, int WPR>
 __global__ __launch_bounds__(kThreads) void rms_norm_kernel(NormArgs a) {
   constexpr int EB = FMT == kFmtF32 ? 4 : 2;
-  const int lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-  if (row >= a.rows) return;
+  constexpr int RPG = kThreads / 64 / WPR;   // rows per workgroup
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t row = (int64_t)blockIdx.x * RPG + wv / WPR;
+  if (row >= a.rows) return;   // whole workgroups where waves share a row (RPG = 1)
   const int chunks = a.hidden / 8;
+  const int ch0 = 64 * (wv % WPR) + lane;
   const char* x = static_cast<const char*>(a.x) + row * a.x_stride * EB;
   const int64_t row_off = row * a.hidden * EB;
-  float h[NC][8], w[NC][8];
+  Raw8<FMT> xr[NC], rr[RES ? NC : 1], wr[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int ch = ch0 + 64 * WPR * c < chunks ? ch0 + 64 * WPR * c : chunks - 1;
+    xr[c] = raw8<FMT>(x + ch * 8 * EB);
+    if constexpr (RES) rr[c] = raw8<FMT>(static_cast<const char*>(a.residual) + row_off + ch * 8 * EB);
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int ch = ch0 + 64 * WPR * c < chunks ? ch0 + 64 * WPR * c : chunks - 1;
+    wr[c] = raw8<FMT>(static_cast<const char*>(a.weight) + ch * 8 * EB);
+  }
+  float h[NC][8];
   float ss = 0.f;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int ch = lane + 64 * c;
-    if (ch >= chunks) continue;
-    load8<FMT>(x + ch * 8 * EB, h[c]);
-    load8<FMT>(static_cast<const char*>(a.weight) + ch * 8 * EB, w[c]);
+    const bool live = ch0 + 64 * WPR * c < chunks;
+    unpack8<FMT>(xr[c], h[c]);
     if constexpr (RES) {
       float r[8];
-      load8<FMT>(static_cast<const char*>(a.residual) + row_off + ch * 8 * EB, r);
+      unpack8<FMT>(rr[c], r);
 #pragma unroll
       for (int e = 0; e < 8; ++e) h[c][e] = round_to<FMT>(__fadd_rn(h[c][e], r[e]));
-      store8<FMT>(static_cast<char*>(a.residual_out) + row_off + ch * 8 * EB, h[c]);
     }
+    if (live) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ss = __fadd_rn(ss, __fmul_rn(h[c][e], h[c][e]));
+      for (int e = 0; e < 8; ++e) ss = __fadd_rn(ss, __fmul_rn(h[c][e], h[c][e]));
+    }
   }
-  const float var = __fmul_rn(wave_sum(ss), a.inv_hidden);
+  ss = wave_sum(ss);
+  if constexpr (WPR > 1) {
+    __shared__ float part[WPR];
+    if (lane == 0) part[wv] = ss;
+    __syncthreads();
+    ss = part[0];
+#pragma unroll
+    for (int w = 1; w < WPR; ++w) ss = __fadd_rn(ss, part[w]);
+  }
+  const float var = __fmul_rn(ss, a.inv_hidden);
   const float rstd = rsqrtf(__fadd_rn(var, a.eps));
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int ch = lane + 64 * c;
+    const int ch = ch0 + 64 * WPR * c;
     if (ch >= chunks) continue;
-    float o[8];
+    if constexpr (RES)
+      store8<FMT>(static_cast<char*>(a.residual_out) + row_off + ch * 8 * EB, h[c]);
+    float w[8], o[8];
+    unpack8<FMT>(wr[c], w);
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-      o[e] = round_to<FMT>(__fmul_rn(w[c][e], round_to<FMT>(__fmul_rn(h[c][e], rstd))));
+      o[e] = round_to<FMT>(__fmul_rn(w[e], round_to<FMT>(__fmul_rn(h[c][e], rstd))));
     store8<FMT>(static_cast<char*>(a.out) + row_off + ch * 8 * EB, o);
   }
 }
@@ -163,21 +221,34 @@ __global__ __launch_bounds__(kThreads) void silu_mul_kernel(SiluArgs a) {
   store8<FMT>(static_cast<char*>(a.out) + (row * a.inter + ch * 8) * EB, o);
 }
 
+// Four waves share a row where a wave alone would hold more than four chunks per lane, and up to
+// kNormSharedRows rows (a decode step's).  us, residual form, bf16, out of cache, four waves /
+// one wave per row / loads between the stores: 9 x 896 2.8 / 2.9 / 3.6, 300 x 896 3.2 / 3.4 /
+// 4.2, 2,736 x 896 6.9 / 6.5 / 6.8, 16 x 3,584 3.3 / 4.6 / 7.0, 700 x 3,584 6.8 / 7.6 / 10.0,
+// 4,096 x 4,096 26.0 (5.2 TB/s) / 30.0 / 30.5.
+constexpr int64_t kNormSharedRows = 256;
+constexpr int kNormSharedHidden = 4 * 64 * 8;   // past it, four chunks per lane of one wave
+
+template <int FMT, bool RES, int WPR>
+int launch_norm_wpr(const NormArgs& a, hipStream_t stream) {
+  const int nc = (a.hidden / 8 + 64 * WPR - 1) / (64 * WPR);
+  constexpr int RPG = kThreads / 64 / WPR;
+  const dim3 grid((unsigned)((a.rows + RPG - 1) / RPG));
+  if (nc <= 1)
+    hipLaunchKernelGGL((rms_norm_kernel<FMT, 1, RES, WPR>), grid, dim3(kThreads), 0, stream, a);
+  else if (nc <= 2)
+    hipLaunchKernelGGL((rms_norm_kernel<FMT, 2, RES, WPR>), grid, dim3(kThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((rms_norm_kernel<FMT, 4, RES, WPR>), grid, dim3(kThreads), 0, stream, a);
+  return check_launch();
+}
+
 template <int FMT, bool RES>
 int launch_norm(const NormArgs& a, hipStream_t stream) {
-  const int nc = (a.hidden / 8 + 63) / 64;
-  const dim3 grid((unsigned)((a.rows + kThreads / 64 - 1) / (kThreads / 64)));
-  if (nc <= 1)
-    hipLaunchKernelGGL((rms_norm_kernel<FMT, 1, RES>), grid, dim3(kThreads), 0, stream, a);
-  else if (nc <= 2)
-    hipLaunchKernelGGL((rms_norm_kernel<FMT, 2, RES>), grid, dim3(kThreads), 0, stream, a);
-  else if (nc <= 4)
-    hipLaunchKernelGGL((rms_norm_kernel<FMT, 4, RES>), grid, dim3(kThreads), 0, stream, a);
-  else if (nc <= 8)
-    hipLaunchKernelGGL((rms_norm_kernel<FMT, 8, RES>), grid, dim3(kThreads), 0, stream, a);
-  else
-    hipLaunchKernelGGL((rms_norm_kernel<FMT, 16, RES>), grid, dim3(kThreads), 0, stream, a);
-  return check_launch();
+  static_assert(kMaxHidden <= 8 * 64 * 4 * 4, "four chunks per lane of four waves");
+  return a.rows <= kNormSharedRows || a.hidden > kNormSharedHidden
+             ? launch_norm_wpr<FMT, RES, 4>(a, stream)
+             : launch_norm_wpr<FMT, RES, 1>(a, stream);
 }
 
 template <int FMT>
