@@ -445,7 +445,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
         valid[t] = v < 0 ? 0 : (v > 16 ? 16 : v);
       }
       // 16-byte chunk c of the stage's V plane: piece c / 64 (t = piece / DT), row (c % 64) / 4
-      for (int c = tid; c < 2 * DT * 64; c += blockDim.x) {
+      for (int c = tid; c < 2 * DT * 64; c += 64 * kPrefWaves) {
         const int piece = c >> 6, row = (c & 63) >> 2;
         if (row >= valid[piece / DT]) st16(&lv[stage][c * 8], u32x4{0u, 0u, 0u, 0u});
       }
@@ -907,7 +907,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     __shared__ int32_t s_n[kPrefSplitTiles], s_at[kPrefSplitTiles];
     __shared__ int32_t s_total;
     const int NQ = a.num_qtiles, tiles = a.num_seqs * NQ;
-    for (int i = tid; i < tiles; i += blockDim.x) {
+    for (int i = tid; i < tiles; i += 64 * kPrefWaves) {
       const int seq = i / NQ;
       PrefTile pt = none;
       pt.seq = seq;
@@ -948,7 +948,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
     int C = (total + a.takers - 1) / a.takers;
     if (C < kPrefMinSteps) C = kPrefMinSteps;
     if (blockIdx.x == 0) {   // the plan, for the merge
-      for (int i = tid; i < tiles; i += blockDim.x) a.ws_plan[2 + i] = s_n[i] > 0 ? s_at[i] : -1;
+      for (int i = tid; i < tiles; i += 64 * kPrefWaves) a.ws_plan[2 + i] = s_n[i] > 0 ? s_at[i] : -1;
       if (tid == 0) {
         a.ws_plan[0] = C;
         a.ws_plan[1] = tiles;
@@ -996,9 +996,9 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
   __shared__ int s_cnt[kPrefListLevels];    // sequences with more than t tiles
   __shared__ int s_off[kPrefListLevels];    // items in the levels above t
   const int S = a.num_seqs, NQ = a.num_qtiles, KVC = a.num_kv_heads;
-  for (int t = tid; t < NQ; t += blockDim.x) s_cnt[t] = 0;
+  for (int t = tid; t < NQ; t += 64 * kPrefWaves) s_cnt[t] = 0;
   lds_barrier();
-  for (int q = tid; q < S; q += blockDim.x) {
+  for (int q = tid; q < S; q += 64 * kPrefWaves) {
     const int64_t t0 = a.cu_seqlens[q];
     int64_t t1 = a.cu_seqlens[q + 1];
     if (t1 > a.num_tokens) t1 = a.num_tokens;
