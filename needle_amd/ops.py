@@ -225,8 +225,10 @@ def decode_workspace_bytes(num_seqs: int, num_heads: int, num_kv_heads: int, hea
     """Bytes of the workspace paged_decode uses for this shape (dtype: of the pool; float32's
     split has a size of its own)."""
     if dtype == torch.float32 and partition_tokens == 0:
-        return int(_lib.load().ndl_paged_decode_f32_workspace_bytes(
+        need = int(_lib.load().ndl_paged_decode_f32_workspace_bytes(
             num_seqs, num_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size))
+        if need:   # 0: a shape the launch refuses, sized (and refused) as the other formats'
+            return need
     return int(_lib.load().ndl_paged_decode_workspace_bytes(
         num_seqs, num_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size,
         partition_tokens))
@@ -579,6 +581,7 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 # tiles) its activations outweigh the weights it streams and the library's GEMM takes over
 # (64 rows, Qwen2-7B gate/up: 69 against 68 us; 32 rows: 60 against 61; 9 rows: 46 against 60).
 SKINNY_ROWS = 64
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
 def skinny_linear_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
@@ -588,7 +591,8 @@ def skinny_linear_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[to
     on the current GPU, k a multiple of 64 and the output columns of 16.  Everything that looks
     at the operation rather than its values (autograd, autocast, tracing, function
     transforms, dispatch modes, tensor subclasses) gets torch's own."""
-    if x.dim() != 2 or not x.is_cuda or not 0 < x.shape[0] <= SKINNY_ROWS:
+    if (type(x) not in _TENSORS or torch.compiler.is_compiling() or x.dim() != 2
+            or not x.is_cuda or not 0 < x.shape[0] <= SKINNY_ROWS):
         return False
     dtype = x.dtype
     if dtype != torch.bfloat16 and dtype != torch.float16:
@@ -611,9 +615,6 @@ def skinny_linear_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[to
             and torch.cuda.current_device() == x.device.index)
 
 
-_TENSORS = (torch.Tensor, torch.nn.Parameter)
-
-
 def _plain(t: torch.Tensor) -> bool:
     """An ordinary tensor in an ordinary call: nothing records, traces or transforms it."""
     return (type(t) in _TENSORS and not (t.requires_grad and torch.is_grad_enabled())
@@ -622,7 +623,7 @@ def _plain(t: torch.Tensor) -> bool:
             and torch._C._functorch.peek_interpreter_stack() is None
             and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._len_torch_function_stack() == 0
-            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+            and not torch.jit.is_tracing())
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor,
