@@ -166,8 +166,11 @@ __global__ __launch_bounds__(64 * NWK * NWR) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           st = __builtin_amdgcn_mfma_f32_16x16x4f32(t.k[m][e], qv[m][e], st, 0, 0, 0);
-      // st[r]: key key0 + r for the lane's row.  Tiles that end at or before the first row's
-      // position need no mask (wave-uniform).
+      // st[r]: key key0 + r for the lane's row, scaled before the mask (-inf times a scale of 0
+      // or less is NaN or +inf).  Tiles that end at or before the first row's position need no
+      // mask (wave-uniform).
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st[r] *= a.scale_log2;
       if (t.bad || tile0 + 16 > (int64_t)ctx + r0 + 1) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -182,10 +185,7 @@ __global__ __launch_bounds__(64 * NWK * NWR) __attribute__((amdgpu_waves_per_eu(
       }
       float mt = kNegInf;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        st[r] *= a.scale_log2;
-        mt = fmaxf(mt, st[r]);
-      }
+      for (int r = 0; r < 4; ++r) mt = fmaxf(mt, st[r]);
       mt = max_xor32(max_xor16(mt));
       const float m_new = fmaxf(m_run, mt);
       const float m_use = m_new == kNegInf ? 0.f : m_new;

@@ -26,9 +26,7 @@ CASES = {
 }
 
 
-@pytest.mark.parametrize("rope", [False, True])
-@pytest.mark.parametrize("name", sorted(CASES))
-def test_prefill_vs_fp64(name, rope):
+def _check(name, rope, scale):
     h, hkv, d, bs, seqs = CASES[name]
     ctx, new = [c for c, _ in seqs], [n for _, n in seqs]
     g = torch.Generator(device=DEV).manual_seed(21)
@@ -51,9 +49,23 @@ def test_prefill_vs_fp64(name, rope):
         more = dict(cos=ang.cos(), sin=ang.sin())
         rot = torch.cat([-q[..., d // 2:], q[..., :d // 2]], -1)
         qr = q * more["cos"][:, None] + rot * more["sin"][:, None]
-    got = ops.varlen_prefill(q, pool, table, cu, lens, max(new), d ** -0.5, h, hkv, d, **more)
-    want = _reference(qr, pool, table, ctx, new, hkv, False)
+    got = ops.varlen_prefill(q, pool, table, cu, lens, max(new), scale * d ** -0.5, h, hkv, d, **more)
+    want = _reference(qr, pool, table, ctx, new, hkv, scale * d ** -0.5)
     keys = max(max(c, 0) + n for c, n in seqs)
     tol = 2 * (keys / 16 + 80) * 2.0 ** -24 * pool.abs().max().item()
     err = (got.double() - want).abs().max().item()
     assert err <= tol, (err, tol)
+
+
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_prefill_vs_fp64(name, rope):
+    _check(name, rope, 1.0)
+
+
+# A masked key stays masked whatever the sign of the scale (-inf times it is NaN or +inf), in
+# both splits of the waves and beside an invalid block.
+@pytest.mark.parametrize("scale", [0.0, -0.0, -1.0])
+@pytest.mark.parametrize("name", ["few", "prefix", "many-even", "uneven"])
+def test_scale_of_any_sign(name, scale):
+    _check(name, False, scale)

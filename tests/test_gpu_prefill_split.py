@@ -27,7 +27,7 @@ CASES = {
 }
 
 
-def _reference(q, pool, table, ctx, new, hkv, bad):
+def _reference(q, pool, table, ctx, new, hkv, scale):
     t, h, d = q.shape
     nb, bs = pool.shape[1], pool.shape[3]
     out = torch.zeros(t, h, d, dtype=torch.float64, device=DEV)
@@ -44,7 +44,7 @@ def _reference(q, pool, table, ctx, new, hkv, bad):
         kv = pool[:, torch.where(ok, blk, 0), :, row % bs].double()   # [keys, 2, hkv, d]
         keys, vals = kv.permute(1, 2, 0, 3).contiguous()
         qi = q[at:at + n].double().view(n, hkv, h // hkv, d).permute(1, 2, 0, 3)
-        w = torch.matmul(qi.reshape(hkv, -1, d), keys.transpose(1, 2).contiguous()) * d ** -0.5
+        w = torch.matmul(qi.reshape(hkv, -1, d), keys.transpose(1, 2).contiguous()) * scale
         w = w.view(hkv, h // hkv, n, c + n)
         mask = (pos > torch.arange(c, c + n, device=DEV)[:, None]) | ~ok
         w = torch.softmax(w.masked_fill(mask, float("-inf")), -1)
@@ -94,7 +94,7 @@ def test_split_equals_whole_tiles(name, rope):
     if rope:
         rot = torch.cat([-q[..., d // 2:], q[..., :d // 2]], -1)
         qr = q * cos[:, None] + rot * sin[:, None]
-    want = _reference(qr, pool, table, ctx, new, hkv, name == "mixed")
+    want = _reference(qr, pool, table, ctx, new, hkv, d ** -0.5)
     ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
     for what, out in (("whole", whole), ("split", got)):
         assert torch.isfinite(out).all(), what
