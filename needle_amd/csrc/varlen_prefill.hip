@@ -81,7 +81,9 @@ struct PrefillArgs {
   const int32_t* context_lens;
   int num_heads;
   int group;          // query heads per kv head
-  float scale_log2;
+  float scale_log2;   // positive: |scale| log2 e
+  uint32_t q_flip;    // 0, or the signs of a word's two elements: q is negated (scale < 0)
+  int q_zero;         // q counts as zeros, scale_log2 is 1 (scale 0)
   int num_qtiles;
   int64_t num_tokens;
   int num_seqs;
@@ -672,11 +674,18 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
       __builtin_amdgcn_wave_barrier();
     }
     {
-      const bool ok = wave_active && wrow0 + r32 < n;
+      const bool ok = wave_active && wrow0 + r32 < n && !a.q_zero;
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         const u32x4 w = *reinterpret_cast<const u32x4*>(&qplane[koff[s]]);
         qb[s] = __builtin_bit_cast(X8, ok ? w : u32x4{0u, 0u, 0u, 0u});
+      }
+      // The softmax scales the masked scores and their max, which takes a positive scale (a
+      // masked -inf times 0 is NaN): the scale's sign goes into q, exactly.
+      if (a.q_flip) {
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+          qb[s] = __builtin_bit_cast(X8, __builtin_bit_cast(u32x4, qb[s]) ^ a.q_flip);
       }
     }
     lds_barrier();
@@ -1290,7 +1299,9 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
   a.context_lens = context_lens;
   a.num_heads = num_heads;
   a.group = group;
-  a.scale_log2 = scale * kLog2e;
+  a.q_zero = scale == 0.f;
+  a.q_flip = scale < 0.f ? 0x80008000u : 0u;
+  a.scale_log2 = a.q_zero ? 1.f : fabsf(scale) * kLog2e;
   a.num_qtiles = (int)qtiles;
   a.num_tokens = num_tokens;
   a.rope_cos = (const u16*)cos;

@@ -54,10 +54,9 @@ def _reference(q, pool, table, ctx, new, hkv, scale):
     return out
 
 
-@pytest.mark.parametrize("rope", [False, True])
-@pytest.mark.parametrize("name", sorted(CASES))
-def test_split_equals_whole_tiles(name, rope):
+def _check(name, rope, scale):
     h, hkv, d, bs, seqs, dtype, cut = CASES[name]
+    scale *= d ** -0.5
     ctx, new = [c for c, _ in seqs], [n for _, n in seqs]
     g = torch.Generator(device=DEV).manual_seed(11)
     width = max(max(-(-(max(c, 0) + n) // bs) for c, n in seqs), 800 // bs) - cut
@@ -80,24 +79,38 @@ def test_split_equals_whole_tiles(name, rope):
     lib = _lib.load()
     code = {torch.bfloat16: 0, torch.float16: 1}[dtype]
     assert lib.ndl_varlen_prefill_workspace_bytes(n_seq, total, max(new), width, h, hkv, d, bs, code)
-    got = ops.varlen_prefill(q, pool, table, cu, lens, max(new), d ** -0.5, h, hkv, d, cos=cos,
+    got = ops.varlen_prefill(q, pool, table, cu, lens, max(new), scale, h, hkv, d, cos=cos,
                              sin=sin)
     whole = torch.empty_like(got)
     rc = lib.ndl_varlen_prefill_split(
         whole.data_ptr(), q.data_ptr(), h * d, cos.data_ptr() if rope else None,
         sin.data_ptr() if rope else None, d, pool.data_ptr(), nb, table.data_ptr(), width, width,
         cu.data_ptr(), lens.data_ptr(), n_seq, total, max(new), 0, h, hkv, d, bs, code,
-        d ** -0.5, None, 0, torch.cuda.current_stream().cuda_stream)
+        scale, None, 0, torch.cuda.current_stream().cuda_stream)
     assert rc == 0
     torch.cuda.synchronize()
     qr = q
     if rope:
         rot = torch.cat([-q[..., d // 2:], q[..., :d // 2]], -1)
         qr = q * cos[:, None] + rot * sin[:, None]
-    want = _reference(qr, pool, table, ctx, new, hkv, d ** -0.5)
+    want = _reference(qr, pool, table, ctx, new, hkv, scale)
     ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
     for what, out in (("whole", whole), ("split", got)):
         assert torch.isfinite(out).all(), what
         err = (out.double() - want).abs() - 2 * ulp * want.abs()
         bad = (err > 2 * ulp).flatten(1).any(1).nonzero().flatten().tolist()
         assert not bad, (what, len(bad), bad[:8], err.max().item())
+
+
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_split_equals_whole_tiles(name, rope):
+    _check(name, rope, 1.0)
+
+
+# A masked key stays masked whatever the sign of the scale (-inf times it is NaN or +inf).
+@pytest.mark.parametrize("scale", [0.0, -0.0, -1.0])
+@pytest.mark.parametrize("name,rope", [("prefix", True), ("one-prompt", False), ("mixed", False),
+                                       ("short-table", True)])
+def test_scale_of_any_sign(name, rope, scale):
+    _check(name, rope, scale)
