@@ -81,9 +81,7 @@ struct PrefillArgs {
   const int32_t* context_lens;
   int num_heads;
   int group;          // query heads per kv head
-  float scale_log2;   // positive: |scale| log2 e
-  uint32_t q_flip;    // 0, or the signs of a word's two elements: q is negated (scale < 0)
-  int q_zero;         // q counts as zeros, scale_log2 is 1 (scale 0)
+  float scale_log2;   // ANY_SCALE: |scale| log2 e, or 1
   int num_qtiles;
   int64_t num_tokens;
   int num_seqs;
@@ -97,6 +95,9 @@ struct PrefillArgs {
   int32_t* ws_plan;   // [2 + tiles]: C, tiles, stream slot of each tile's first step
   float* ws_ml;       // [slot][wave][lane][2] = (m, l)
   float* ws_acc;      // [slot][wave][accumulator quad][lane][4]
+  // ANY_SCALE
+  uint32_t q_flip;    // the signs of a word's two elements, flipped in q (scale < 0)
+  int q_zero;         // q counts as zeros (scale 0)
 };
 
 // One workgroup tile, looked up one tile ahead by the persistent walk: jobs
@@ -153,7 +154,12 @@ __device__ __forceinline__ float half_sum(float v) {
 // registers (with the reference's rounding, rope8), from cos/sin rows of its token.
 // F16: the elements are fp16 (else bf16).
 // SPLIT: the launch of prefill_split_kernel (below).
-template <int D, int NS, bool ROPE, bool F16, bool SPLIT>
+// ANY_SCALE: scales of 0 or less.  The softmax scales masked scores (-inf) and the row's raw
+// maximum, which is right for a positive scale only (-inf times 0 is NaN), so the scale's sign
+// goes into q, exactly, and a scale of 0 counts q as zeros.  A form of its own: one uniform
+// branch per tile cost the positive scales 1.2% (137.8 -> 139.4 us, 16 prompts of 128 to 2,048
+// tokens, 28/4 heads of 128).
+template <int D, int NS, bool ROPE, bool F16, bool SPLIT, bool ANY_SCALE>
 __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
   using T = Elt<F16>;
   using X8 = typename T::x8;
@@ -674,17 +680,13 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
       __builtin_amdgcn_wave_barrier();
     }
     {
-      const bool ok = wave_active && wrow0 + r32 < n && !a.q_zero;
+      bool ok = wave_active && wrow0 + r32 < n;
+      if constexpr (ANY_SCALE) ok = ok && !a.q_zero;
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         const u32x4 w = *reinterpret_cast<const u32x4*>(&qplane[koff[s]]);
         qb[s] = __builtin_bit_cast(X8, ok ? w : u32x4{0u, 0u, 0u, 0u});
-      }
-      // The softmax scales the masked scores and their max, which takes a positive scale (a
-      // masked -inf times 0 is NaN): the scale's sign goes into q, exactly.
-      if (a.q_flip) {
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
+        if constexpr (ANY_SCALE)
           qb[s] = __builtin_bit_cast(X8, __builtin_bit_cast(u32x4, qb[s]) ^ a.q_flip);
       }
     }
@@ -1108,7 +1110,11 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a) {
 
 template <int D, int NS, bool ROPE, bool F16>
 __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(PrefillArgs a) {
-  prefill_body<D, NS, ROPE, F16, false>(a);
+  prefill_body<D, NS, ROPE, F16, false, false>(a);
+}
+template <int D, int NS, bool ROPE, bool F16>
+__global__ __launch_bounds__(64 * kPrefWaves) void prefill_any_scale_kernel(PrefillArgs a) {
+  prefill_body<D, NS, ROPE, F16, false, true>(a);
 }
 
 // The same tiles with their keys split over the workgroups: each takes the same number of
@@ -1116,7 +1122,7 @@ __global__ __launch_bounds__(64 * kPrefWaves) void varlen_prefill_kernel(Prefill
 // that prefill_merge_kernel adds.
 template <int D, int NS, bool ROPE, bool F16>
 __global__ __launch_bounds__(64 * kPrefWaves) void prefill_split_kernel(PrefillArgs a) {
-  prefill_body<D, NS, ROPE, F16, true>(a);
+  prefill_body<D, NS, ROPE, F16, true, false>(a);
 }
 
 // One workgroup per (query tile, kv head, 32 columns of head_dim), wave w its job w: adds the tile's partials in
@@ -1186,19 +1192,20 @@ __global__ __launch_bounds__(64 * kPrefWaves) void prefill_merge_kernel(PrefillA
 
 namespace ndl {
 
-inline const void* prefill_split_fn(int head_dim, bool f16, bool rope) {
-  // [f16][head_dim 128][rope]
-  const void* const fns[2][2][2] = {
-      {{(const void*)prefill_split_kernel<64, 8, false, false>,
-        (const void*)prefill_split_kernel<64, 8, true, false>},
-       {(const void*)prefill_split_kernel<128, 6, false, false>,
-        (const void*)prefill_split_kernel<128, 6, true, false>}},
-      {{(const void*)prefill_split_kernel<64, 8, false, true>,
-        (const void*)prefill_split_kernel<64, 8, true, true>},
-       {(const void*)prefill_split_kernel<128, 6, false, true>,
-        (const void*)prefill_split_kernel<128, 6, true, true>}}};
-  return fns[f16 ? 1 : 0][head_dim == 128 ? 1 : 0][rope ? 1 : 0];
-}
+// The instantiation of a kernel for one call.
+#define NDL_PREFILL_FN(name, kernel)                                                        \
+  inline const void* name(int head_dim, bool f16, bool rope) {                              \
+    const void* const fns[2][2][2] = { /* [f16][head_dim 128][rope] */                      \
+        {{(const void*)kernel<64, 8, false, false>, (const void*)kernel<64, 8, true, false>}, \
+         {(const void*)kernel<128, 6, false, false>, (const void*)kernel<128, 6, true, false>}}, \
+        {{(const void*)kernel<64, 8, false, true>, (const void*)kernel<64, 8, true, true>},   \
+         {(const void*)kernel<128, 6, false, true>, (const void*)kernel<128, 6, true, true>}}}; \
+    return fns[f16 ? 1 : 0][head_dim == 128 ? 1 : 0][rope ? 1 : 0];                         \
+  }
+NDL_PREFILL_FN(prefill_fn, varlen_prefill_kernel)
+NDL_PREFILL_FN(prefill_any_scale_fn, prefill_any_scale_kernel)
+NDL_PREFILL_FN(prefill_split_fn, prefill_split_kernel)
+#undef NDL_PREFILL_FN
 
 // The split launch's layout, or false where whole tiles are taken.  Whole tiles take as long
 // as the longest one, split ones the average over the GPU plus about 40 steps (a second ring
@@ -1299,6 +1306,7 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
   a.context_lens = context_lens;
   a.num_heads = num_heads;
   a.group = group;
+  const bool any_scale = !(scale > 0.f);
   a.q_zero = scale == 0.f;
   a.q_flip = scale < 0.f ? 0x80008000u : 0u;
   a.scale_log2 = a.q_zero ? 1.f : fabsf(scale) * kLog2e;
@@ -1316,7 +1324,7 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
                  gx * (int64_t)num_seqs * qtiles < ((int64_t)1 << 31);
   const bool f16 = dtype_is_f16(dtype);
   PrefillSplit sp;
-  if (workspace != nullptr && ((uintptr_t)workspace & 15u) == 0 &&
+  if (workspace != nullptr && ((uintptr_t)workspace & 15u) == 0 && !any_scale &&
       prefill_split(num_seqs, num_tokens, qtiles, num_heads, num_kv_heads, head_dim, a.max_tiles,
                     &sp) &&
       workspace_bytes >= sp.bytes) {
@@ -1345,17 +1353,8 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
     }
     return check_launch();
   }
-  // [f16][head_dim 128][rope]
-  const void* const fns[2][2][2] = {
-      {{(const void*)varlen_prefill_kernel<64, 8, false, false>,
-        (const void*)varlen_prefill_kernel<64, 8, true, false>},
-       {(const void*)varlen_prefill_kernel<128, 6, false, false>,
-        (const void*)varlen_prefill_kernel<128, 6, true, false>}},
-      {{(const void*)varlen_prefill_kernel<64, 8, false, true>,
-        (const void*)varlen_prefill_kernel<64, 8, true, true>},
-       {(const void*)varlen_prefill_kernel<128, 6, false, true>,
-        (const void*)varlen_prefill_kernel<128, 6, true, true>}}};
-  const void* fn = fns[f16 ? 1 : 0][head_dim == 128 ? 1 : 0][rope ? 1 : 0];
+  const void* const fn = any_scale ? prefill_any_scale_fn(head_dim, f16, rope)
+                                   : prefill_fn(head_dim, f16, rope);
   dim3 grid((unsigned)gx, (unsigned)num_seqs, (unsigned)qtiles);
   if (a.persistent) {
     const int64_t slots = resident_workgroups(fn, 64 * waves);
