@@ -124,6 +124,61 @@ __device__ __forceinline__ int64_t stream_chunk(const DecodeArgs& a, int lane) {
   return stream_chunk_of(a, total);
 }
 
+// What one pass over the context lengths gives (longest: per lane, of the sequences it saw).
+struct StreamSizes {
+  int64_t slots;   // of the stream
+  int seqs;        // sequences with something to attend
+  int longest;     // tiles
+};
+__device__ __forceinline__ void add_sizes(StreamSizes& z, int n) {
+  z.seqs += __builtin_popcountll(__builtin_amdgcn_ballot_w64(n > 0));
+  z.longest = n > z.longest ? n : z.longest;
+}
+
+// Whether the float32 stream's workgroups take whole sequences instead of equal shares (its
+// attention kernel and its merge both ask).  Equal shares end the wait for the longest sequence
+// and cost a second start per workgroup, the partials and the merge; only the lengths tell, and
+// only the device knows those (the table may be much wider).  Whole sequences where the longest
+// has at most f32_short_tiles, or, while each (kv head, sequence) has a workgroup of its own, at
+// most a third more than an equal share (and, at head_dim 64, f32_spare_tiles, what the second
+// start and the merge take there).  us per launch pair, equal shares / whole / one launch per
+// sequence (a 16-tile table): tables of 256 columns, 14/2 heads of 64, 8 sequences of 100 tokens
+// 13.9 / 9.4 / 7.5, 400 14.1 / 12.6, 500 13.8 / 13.4; 28/4 of 128, 100 17.7 / 13.5 / 11.8, 300
+// 18.4 / 18.1 / 16.1, 400 18.8 / 21.8.  Even batches: 32/8 heads, 32 of 1,000 60.9 / 58.7; 32/32,
+// 8 of 1,000 58.9 / 57.2; 28/4, 48 of 1,000 53.9 / 47.3; uneven ones keep equal shares (32 of 104
+// to 3,936, 28/4 heads, 44 / 104).
+template <int D> constexpr int f32_short_tiles() { return D == 64 ? 28 : 18; }
+template <int D> constexpr int f32_spare_tiles() { return D == 64 ? 24 : 0; }
+// n: the lane's tiles of the first 64 sequences.  Asked before anything else is computed: short
+// sequences are over in the time it takes.
+template <int D>
+__device__ __forceinline__ bool f32_all_short(const DecodeArgs& a, int n) {
+  return a.num_seqs <= 64 && __builtin_amdgcn_ballot_w64(n > f32_short_tiles<D>()) == 0;
+}
+template <int D>
+__device__ __forceinline__ bool f32_takes_whole(const DecodeArgs& a, const StreamSizes& z) {
+  int64_t most = f32_short_tiles<D>();
+  if (z.seqs <= a.waves) {
+    const int64_t share = z.slots * 4 / (3 * (int64_t)a.waves) + f32_spare_tiles<D>();
+    most = share > most ? share : most;
+  }
+  return __builtin_amdgcn_ballot_w64(z.longest > most) == 0;
+}
+// The sizes of a stream whose workgroups take equal shares, or nothing (false) where they take
+// whole sequences.
+template <int D, int PAD>
+__device__ __forceinline__ bool f32_shares(const DecodeArgs& a, int lane, StreamSizes* z) {
+  *z = StreamSizes{0, 0, 0};
+  for (int base = 0; base < a.num_seqs; base += 64) {
+    const int q = base + lane;
+    const int n = q < a.num_seqs ? seq_tiles(a, q) : 0;
+    if (base == 0 && f32_all_short<D>(a, n)) return false;
+    z->slots += __builtin_amdgcn_readlane(wave_incl_scan(stream_slots<PAD>(n), lane), 63);
+    add_sizes(*z, n);
+  }
+  return !f32_takes_whole<D>(a, *z);
+}
+
 // Merge of the segment partials: MW waves per (query head, sequence).  A sequence
 // whose tiles lie with takers s0 .. s1 of its kv head's stream has its partials in
 // segment slots s0 + seq .. s1 + seq; a sequence inside one taker was written by the
@@ -148,7 +203,8 @@ __global__ __launch_bounds__(64 * MW) void paged_decode_merge_kernel(DecodeArgs 
   // it from registers; the first query head's wave of each (kv head, sequence) stores it,
   // with the separate append's rule (attention.py:141-154): column min(ctx / bs, W - 1),
   // row ctx % bs, nothing for a negative context or an invalid block id.
-  if (a.k_new != nullptr && hc == 0 && wv == 0) {
+  auto store_row = [&] {
+    if (a.k_new == nullptr || hc != 0 || wv != 0) return;
     constexpr int EC = 16 / EB;  // elements per 16-byte chunk
     constexpr int CH = D / EC;   // 16-byte chunks per row; lanes < CH: K, < 2 CH: V
     static_assert(2 * CH <= 64, "a lane per chunk of the two rows");
@@ -183,7 +239,7 @@ __global__ __launch_bounds__(64 * MW) void paged_decode_merge_kernel(DecodeArgs 
         st16(row, val);
       }
     }
-  }
+  };
   char* dst = (char*)a.out + (((int64_t)seq * a.num_heads + head) * D + lane * PER_LANE) * EB;
   auto store_out = [&](const float (&o)[PER_LANE]) {
     if constexpr (FMT == kFmtF32) {
@@ -202,27 +258,42 @@ __global__ __launch_bounds__(64 * MW) void paged_decode_merge_kernel(DecodeArgs 
   float acc[PER_LANE];
 #pragma unroll
   for (int e = 0; e < PER_LANE; ++e) acc[e] = 0.f;
-  // One pass over context_lens (one load per 64 sequences, nothing else in flight before
-  // it): this sequence's tiles, its first stream tile and the stream's total, i.e. what
-  // seq_tiles, stream_locate and stream_chunk give.
+  // One pass over context_lens (one load per 64 sequences): this sequence's tiles, its first
+  // stream tile and the stream's sizes, i.e. what seq_tiles, stream_locate and stream_sizes give.
   int nt = 0;
-  int64_t first = 0, total = 0;
-  for (int base = 0; base < a.num_seqs; base += 64) {
-    const int q = base + lane;
-    const int n = q < a.num_seqs ? seq_tiles(a, q) : 0;
-    const int v = stream_slots<PAD>(n);
-    const int incl = wave_incl_scan(v, lane);
-    if (seq >= base && seq < base + 64) {   // the sequence's tile count and first tile
-      nt = __builtin_amdgcn_readlane(n, seq - base);
-      first = total + __builtin_amdgcn_readlane(incl - v, seq - base) + PAD;
+  int64_t first = 0;
+  StreamSizes z{0, 0, 0};
+  auto scan = [&] {   // false: the sequences' workgroups wrote everything (float32)
+    for (int base = 0; base < a.num_seqs; base += 64) {
+      const int q = base + lane;
+      const int n = q < a.num_seqs ? seq_tiles(a, q) : 0;
+      if constexpr (FMT == kFmtF32) {
+        if (base == 0 && f32_all_short<D>(a, n)) return false;
+      }
+      const int v = stream_slots<PAD>(n);
+      const int incl = wave_incl_scan(v, lane);
+      if (seq >= base && seq < base + 64) {   // the sequence's tile count and first tile
+        nt = __builtin_amdgcn_readlane(n, seq - base);
+        first = z.slots + __builtin_amdgcn_readlane(incl - v, seq - base) + PAD;
+      }
+      z.slots += __builtin_amdgcn_readlane(incl, 63);
+      if constexpr (FMT == kFmtF32) add_sizes(z, n);
     }
-    total += __builtin_amdgcn_readlane(incl, 63);
+    if constexpr (FMT == kFmtF32) return !f32_takes_whole<D>(a, z);
+    return true;
+  };
+  if constexpr (FMT == kFmtF32) {
+    if (!scan()) return;
+    store_row();
+  } else {
+    store_row();
+    scan();
   }
   if (nt == 0) {
     if (wv == 0) store_out(acc);
     return;
   }
-  const int64_t chunk = stream_chunk_of(a, total);
+  const int64_t chunk = stream_chunk_of(a, z.slots);
   const int64_t s0 = first / chunk, s1 = (first + nt - 1) / chunk;
   if (s0 == s1) return;
   const int nparts = (int)(s1 - s0 + 1);

@@ -12,9 +12,10 @@
 // longest sequence on a fraction of the GPU: 12 sequences of up to 4,000 tokens, 4 kv heads,
 // 87 us per layer at 0.56 TB/s.  With a workspace the tiles of all sequences are one stream
 // (decode_stream.hpp) shared by as many workgroups as can be resident, each taking the
-// same number of tiles, and a merge adds the partials: 26.5 us, 1.84 TB/s; what is left is the
-// start of each workgroup and the merge (14 us for a single tile per wave).  The products run on v_mfma_f32_16x16x4_f32 (fp32
-// operands, fp32 accumulation), the probabilities stay fp32:
+// same number of tiles, and a merge adds the partials: 26.1 us, 1.87 TB/s; what is left is the
+// start of each workgroup and the merge (14 us for a single tile per wave).  Where the lengths are short or even the workgroups
+// take whole sequences after all (f32_takes_whole).  The products run on v_mfma_f32_16x16x4_f32
+// (fp32 operands, fp32 accumulation), the probabilities stay fp32:
 //   * S^T = K q^T: M = the tile's 16 tokens, N = the g query heads (padded to 16),
 //     K = head_dim in steps of 4.  Lane (i, kk) = (lane % 16, lane / 16) holds
 //     K[token i][16 m + 4 kk + e] and q[head i][16 m + 4 kk + e] for m < D/16, e < 4 (one
@@ -32,6 +33,8 @@
 // in the same call, as the 16-bit kernel does; q is rotated as it is loaded.
 #include "decode_stream.hpp"
 
+#include <type_traits>
+
 namespace ndl {
 
 constexpr int kF32Waves = 8;
@@ -47,10 +50,21 @@ __device__ __forceinline__ f32x4 ldf4(const float* p) {
   return *reinterpret_cast<const f32x4*>(p);
 }
 
+// The launch's arguments, read again where they are used: what a rare path needs (the step's
+// row, the output) then holds no scalar registers through the walk.
+typedef const __attribute__((address_space(4))) DecodeArgs DecodeArgsConst;
+__device__ __forceinline__ DecodeArgsConst& fresh_args() {
+  DecodeArgsConst* p = (DecodeArgsConst*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *p;
+}
+
 // SPLIT: workgroup sw of a kv head takes stream slots sw*C .. sw*C + C, whatever sequences
-// they belong to; otherwise one workgroup per (kv head, sequence).  APP: the step's row
-// (a.k_new, a.v_new) is attended in place of the pool's stale one; without SPLIT the wave that
-// attends it also stores it, with SPLIT the merge kernel does.
+// they belong to, or the whole sequences sw, sw + takers, .. where the lengths make that the
+// faster one (f32_takes_whole); otherwise one workgroup per (kv head, sequence).  APP: the
+// step's row (a.k_new, a.v_new) is attended in place of the pool's stale one; where a workgroup
+// has the whole sequence the wave that attends the row also stores it, else the merge kernel
+// does.
 template <int D, bool ROPE, bool APP, bool SPLIT>
 __global__ __launch_bounds__(64 * kF32Waves) void paged_decode_f32_kernel(DecodeArgs a) {
   constexpr int NW = kF32Waves;
@@ -73,12 +87,22 @@ __global__ __launch_bounds__(64 * kF32Waves) void paged_decode_f32_kernel(Decode
   const float* const vplane = (const float*)a.vplane;
   __shared__ __attribute__((aligned(16))) float sacc[NW * E * 64];
   __shared__ float sm[NW * 16], sl[NW * 16];
+  // The split form at head_dim 128 has no registers to spare: with its arguments held it spilled
+  // to memory (32 of 1,000 tokens as whole sequences, 28/4 heads: 45.7 us, read again 41.2).
+  auto args = [&]() -> decltype(auto) {
+    if constexpr (SPLIT && D == 128)
+      return fresh_args();
+    else
+      return (a);
+  };
   bool smem_busy = false;   // an earlier piece's combine may still be reading LDS
 
   // Tiles lt0 .. lt1 of sequence seq (n_tiles in all), the waves taking every NW-th; every
-  // wave of the workgroup calls it together (it has barriers).
-  auto piece = [&](const int seq, const int lt0, const int lt1, const int n_tiles,
+  // wave of the workgroup calls it together (it has barriers).  whole_seq: std::true_type where
+  // these are all its tiles.
+  auto piece = [&](auto whole_seq, const int seq, const int lt0, const int lt1, const int n_tiles,
                    const int segid) {
+    constexpr bool WHOLE = decltype(whole_seq)::value;
     const int64_t L = attended_len(a, seq);
     const int first = lt0 + wv;
     const int ntw = first < lt1 ? (lt1 - first + NW - 1) / NW : 0;   // this wave's tiles
@@ -97,14 +121,15 @@ __global__ __launch_bounds__(64 * kF32Waves) void paged_decode_f32_kernel(Decode
     // q^T operand (lanes past the group read the group's first head and zero it)
     f32x4 qv[QK];
     {
-      const float* qrow = (const float*)a.q + (int64_t)seq * a.q_tok_stride +
+      auto&& r = args();
+      const float* qrow = (const float*)r.q + (int64_t)seq * r.q_tok_stride +
                           (int64_t)(head_ok ? head : kvh * a.group) * D + 4 * kk;
 #pragma unroll
       for (int m = 0; m < QK; ++m) qv[m] = ldf4(qrow + 16 * m);
       if constexpr (ROPE) {
         // element 16 m + 4 kk + e pairs with the same lane's piece m + QK / 2
-        const float* crow = (const float*)a.rope_cos + (int64_t)seq * a.rope_stride + 4 * kk;
-        const float* srow = (const float*)a.rope_sin + (int64_t)seq * a.rope_stride + 4 * kk;
+        const float* crow = (const float*)r.rope_cos + (int64_t)seq * r.rope_stride + 4 * kk;
+        const float* srow = (const float*)r.rope_sin + (int64_t)seq * r.rope_stride + 4 * kk;
 #pragma unroll
         for (int m = 0; m < QK / 2; ++m) {
           u32x4 lo, hi;
@@ -164,16 +189,17 @@ __global__ __launch_bounds__(64 * kF32Waves) void paged_decode_f32_kernel(Decode
       // The step's row in place of row r_new of its tile (loaded where it is used: one tile
       // of one wave per sequence, and its registers are not held through the walk).
       auto put_new_row = [&](Tile& t) {
-        const float* krow = (const float*)a.k_new + (int64_t)seq * a.k_new_stride +
+        auto&& r = args();
+        const float* krow = (const float*)r.k_new + (int64_t)seq * r.k_new_stride +
                             (int64_t)kvh * D + 4 * kk;
-        const float* vrow = (const float*)a.v_new + (int64_t)seq * a.v_new_stride +
+        const float* vrow = (const float*)r.v_new + (int64_t)seq * r.v_new_stride +
                             (int64_t)kvh * D + 4 * i16;
         f32x4 kn[QK];
 #pragma unroll
         for (int m = 0; m < QK; ++m) kn[m] = ldf4(krow + 16 * m);
         if constexpr (ROPE) {
-          const float* crow = (const float*)a.rope_cos + (int64_t)seq * a.rope_stride + 4 * kk;
-          const float* srow = (const float*)a.rope_sin + (int64_t)seq * a.rope_stride + 4 * kk;
+          const float* crow = (const float*)r.rope_cos + (int64_t)seq * r.rope_stride + 4 * kk;
+          const float* srow = (const float*)r.rope_sin + (int64_t)seq * r.rope_stride + 4 * kk;
 #pragma unroll
           for (int m = 0; m < QK / 2; ++m) {
             u32x4 lo, hi;
@@ -189,8 +215,8 @@ __global__ __launch_bounds__(64 * kF32Waves) void paged_decode_f32_kernel(Decode
         if (i16 == r_new) {
 #pragma unroll
           for (int m = 0; m < QK; ++m) t.k[m] = kn[m];
-          if constexpr (!SPLIT) {
-            float* const kd = const_cast<float*>(kplane) + t.off + (int64_t)r_new * D + 4 * kk;
+          if constexpr (WHOLE) {
+            float* const kd = (float*)r.kplane + t.off + (int64_t)r_new * D + 4 * kk;
 #pragma unroll
             for (int m = 0; m < QK; ++m) *reinterpret_cast<f32x4*>(kd + 16 * m) = kn[m];
           }
@@ -201,9 +227,9 @@ __global__ __launch_bounds__(64 * kF32Waves) void paged_decode_f32_kernel(Decode
 #pragma unroll
           for (int t4 = 0; t4 < 4; ++t4)
             if (4 * kk + t4 == r_new) t.v[g][t4] = vn;
-          if constexpr (!SPLIT) {
+          if constexpr (WHOLE) {
             if (kk == r_new >> 2)
-              *reinterpret_cast<f32x4*>(const_cast<float*>(vplane) + t.off + (int64_t)r_new * D +
+              *reinterpret_cast<f32x4*>((float*)r.vplane + t.off + (int64_t)r_new * D +
                                         4 * i16 + 64 * g) = vn;
           }
         }
@@ -311,17 +337,18 @@ __global__ __launch_bounds__(64 * kF32Waves) void paged_decode_f32_kernel(Decode
     const int x0 = wv * KPW;
     const int g = x0 / 16, r = (x0 / 4) % 4, e0 = x0 % 4;
     const int d0 = 64 * g + 16 * kk + 4 * r + e0;
+    auto&& y = args();
     float* dst;
     float inv = 1.f;
-    if (!SPLIT || (lt0 == 0 && lt1 == n_tiles)) {   // the whole sequence: final output
+    if (WHOLE || (lt0 == 0 && lt1 == n_tiles)) {   // the whole sequence: final output
       inv = den > 0.f ? 1.f / den : 0.f;
-      dst = (float*)a.out + ((int64_t)seq * a.num_heads + head) * D + d0;
+      dst = (float*)y.out + ((int64_t)seq * y.num_heads + head) * D + d0;
     } else {
-      const int64_t slot = ((int64_t)kvh * a.nseg + segid) * a.group + i16;
-      dst = a.ws_acc + slot * D + d0;
+      const int64_t slot = ((int64_t)kvh * y.nseg + segid) * a.group + i16;
+      dst = y.ws_acc + slot * D + d0;
       if (wv == 0 && kk == 0) {
-        a.ws_ml[slot * 2] = mx;
-        a.ws_ml[slot * 2 + 1] = den;
+        y.ws_ml[slot * 2] = mx;
+        y.ws_ml[slot * 2 + 1] = den;
       }
     }
     if constexpr (KPW == 4) {
@@ -334,9 +361,17 @@ __global__ __launch_bounds__(64 * kF32Waves) void paged_decode_f32_kernel(Decode
 
   if constexpr (!SPLIT) {
     const int nt = seq_tiles(a, sw);
-    piece(sw, 0, nt, nt, 0);
+    piece(std::true_type{}, sw, 0, nt, nt, 0);
   } else {
-    const int64_t chunk = stream_chunk<kF32StreamPad>(a, lane);
+    StreamSizes sizes;
+    if (!f32_shares<D, kF32StreamPad>(a, lane, &sizes)) {
+      for (int seq = sw; seq < a.num_seqs; seq += a.waves) {
+        const int nt = seq_tiles(a, seq);
+        piece(std::true_type{}, seq, 0, nt, nt, 0);
+      }
+      return;
+    }
+    const int64_t chunk = stream_chunk_of(a, sizes.slots);
     const int64_t start = (int64_t)sw * chunk, end = start + chunk;
     int seq;
     int64_t at;
@@ -347,7 +382,8 @@ __global__ __launch_bounds__(64 * kF32Waves) void paged_decode_f32_kernel(Decode
         const int64_t t0 = at + kF32StreamPad;   // the sequence's first tile
         const int64_t s0 = start > t0 ? start : t0;
         const int64_t s1 = end < t0 + nt ? end : t0 + nt;
-        if (s1 > s0) piece(seq, (int)(s0 - t0), (int)(s1 - t0), nt, sw + seq);
+        if (s1 > s0)
+          piece(std::false_type{}, seq, (int)(s0 - t0), (int)(s1 - t0), nt, sw + seq);
       }
       at += stream_slots<kF32StreamPad>(nt);
       ++seq;
@@ -369,7 +405,8 @@ const void* decode_f32_split_fn(bool rope, bool app) {
 }
 template <int D>
 const void* decode_f32_seq_fn(bool rope, bool app) {
-  return rope ? (const void*)paged_decode_f32_kernel<D, true, true, false>
+  return rope ? (app ? (const void*)paged_decode_f32_kernel<D, true, true, false>
+                     : (const void*)paged_decode_f32_kernel<D, true, false, false>)
               : app ? (const void*)paged_decode_f32_kernel<D, false, true, false>
                     : (const void*)paged_decode_f32_kernel<D, false, false, false>;
 }
@@ -390,17 +427,33 @@ static DecodeF32Layout decode_f32_layout(int num_seqs, int num_heads, int num_kv
   return lay;
 }
 
-// Most tiles of a table row for which one workgroup per (kv head, sequence) is taken: up to
-// here the merge launch costs what the split gains.  us split / whole, 8 sequences: head_dim 64
-// (2 kv heads) at 32 tiles 14.7 / 11.8, 48 15.3 / 14.9, 63 14.4 / 18.0, 125 18.0 / 29.6, 250
-// 18.1 / 51; head_dim 128 (4 kv heads) at 16 21.3 / 15.3, 32 21.7 / 21.9, 48 22.0 / 27.7, 63
-// 21.3 / 34, 250 40 / 102.  Equal sequences that fill the GPU by themselves (32 of 4,000 tokens,
-// 8 kv heads) 194.5 / 189.5; unequal ones gain there too.
-template <int D> constexpr int f32_seq_max_tiles() { return D == 64 ? 48 : 32; }
+// Whether a table may be long enough to split (two launches; the lengths then decide on the
+// device, f32_takes_whole): up to here one launch of one workgroup per (kv head, sequence) costs
+// less whatever the lengths are.  us split / whole, 8 sequences: head_dim 64 (2 kv heads) at 32
+// tiles 14.7 / 11.8, 48 15.3 / 14.9, 63 14.4 / 18.0, 125 18.0 / 29.6, 250 18.1 / 51; head_dim 128
+// (4 kv heads) at 16 21.3 / 15.3, 32 21.7 / 21.9, 48 22.0 / 27.7, 63 21.3 / 34, 250 40 / 102.
+// Pairs that fill most of the GPU gain nothing from a split of short sequences: 14/2 heads of 64,
+// 128 sequences of 85 to 996 tokens 24.2 / 20.5, 64 of 1,000 22.5 / 19.3; 28/4 of 128, 64 of 600
+// 42.4 / 38.3, 48 of 122 to 595 28.8 / 26.8 (63 tiles, 48 of 86 to 989: 33.2 / 37.5), and from
+// two workgroups per CU 128 of 302 to 599 68.3 / 61.1, 32/32 heads, 16 of 1,000 110 / 102.5.
+static bool f32_split_takes(int num_seqs, int num_kv_heads, int head_dim, int64_t max_tiles) {
+  const int64_t pairs = (int64_t)num_seqs * num_kv_heads;
+  if (head_dim == 64) return max_tiles > (pairs >= 128 && pairs <= 256 ? 64 : 48);
+  return max_tiles > (pairs >= 512 ? 64 : pairs >= 192 && pairs <= 256 ? 40 : 32);
+}
+
+// Batches whose rows are appended by a launch of their own before whole sequences are attended:
+// the wave that attends a row it is given finishes later, which three rounds of workgroups wait
+// for three times.  us in one launch / two: 100 sequences of 51 to 498 tokens, 32/8 heads of 128,
+// 63.7 / 61.3, 32/32 196 / 184; 128 of 300 32/32 302 / 281; 64 of 600 264 / 256; but 32 of 100 to
+// 199 57 / 61, 24 of 504 to 996 118 / 128, and 16 of 400 52 / 62.
+static bool f32_append_first(int num_seqs, int num_kv_heads) {
+  return num_seqs >= 64 && (int64_t)num_seqs * num_kv_heads >= 768;
+}
 
 size_t decode_f32_workspace_bytes(int num_seqs, int num_heads, int num_kv_heads, int head_dim,
                                   int64_t max_tiles) {
-  if (max_tiles <= (head_dim == 128 ? f32_seq_max_tiles<128>() : f32_seq_max_tiles<64>())) return 256;
+  if (!f32_split_takes(num_seqs, num_kv_heads, head_dim, max_tiles)) return 256;
   return decode_f32_layout(num_seqs, num_heads, num_kv_heads, head_dim).bytes;
 }
 
@@ -445,11 +498,12 @@ int launch_decode_f32(void* out, const void* q, int64_t q_tok_stride, const void
   a.rope_cos = (const u16*)cos;
   a.rope_sin = (const u16*)sin;
   a.rope_stride = cs_tok_stride;
-  const bool rope = cos != nullptr, app = k_new != nullptr;
+  const bool rope = cos != nullptr;
+  bool app = k_new != nullptr;
   hipStream_t s = (hipStream_t)stream;
   const int64_t max_tiles = (int64_t)max_blocks_per_seq << a.tile_shift;
   bool split = false;
-  if (max_tiles > (head_dim == 128 ? f32_seq_max_tiles<128>() : f32_seq_max_tiles<64>()) && workspace != nullptr &&
+  if (f32_split_takes(num_seqs, num_kv_heads, head_dim, max_tiles) && workspace != nullptr &&
       ((uintptr_t)workspace & 15u) == 0) {
     const DecodeF32Layout lay = decode_f32_layout(num_seqs, num_heads, num_kv_heads, head_dim);
     split = workspace_bytes >= lay.bytes && lay.nseg <= 0x7fffffff;
@@ -457,6 +511,14 @@ int launch_decode_f32(void* out, const void* q, int64_t q_tok_stride, const void
     a.nseg = (int)lay.nseg;
     a.ws_ml = (float*)workspace;
     a.ws_acc = (float*)((char*)workspace + lay.ml_bytes);
+  }
+  if (app && !split && f32_append_first(num_seqs, num_kv_heads)) {
+    const int rc = launch_kv_append(kv_cache, num_blocks, num_kv_heads, block_size, head_dim,
+                                    k_new, k_tok_stride, v_new, v_tok_stride, block_table,
+                                    bt_row_stride, max_blocks_per_seq, nullptr, context_lens,
+                                    num_seqs, num_seqs, cos, sin, cs_tok_stride, kFmtF32, stream);
+    if (rc != NDL_OK) return rc;
+    app = false;
   }
   const void* fn = split ? (head_dim == 128 ? decode_f32_split_fn<128>(rope, app)
                                             : decode_f32_split_fn<64>(rope, app))
