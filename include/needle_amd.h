@@ -357,11 +357,16 @@ int ndl_rope_varlen_prefill(void* out, const void* q, int64_t q_tok_stride,
  * aligned (calls that share one must not overlap): where few query tiles attend many keys
  * (a prompt after a long cached prefix, one long prompt), the keys of each tile are split over
  * workgroups and the pieces merged, in two launches.  Results differ by the order of the fp32
- * sums.  workspace NULL or too small, or a shape of 0 bytes: as those entry points.
+ * sums.  The choice counts max_context_len + max_seqlen keys (at most the table's): with
+ * max_context_len 0 after a cached prefix the result is right and the tiles stay whole.
+ * workspace NULL or too small, a scale of 0 or less, or a shape of 0 bytes: as those entry points.
+ *
+ * ndl_varlen_prefill_workspace_bytes takes as max_blocks_per_seq the smaller of the table's
+ * columns and the blocks of max_context_len + max_seqlen tokens.
  *
  * Replaces: needle/layers/attention.py:120-134 (_prefill_pytorch).
  */
-#define NDL_PREFILL_SPLIT_MIN_KEYS 768   /* 0 bytes for tables of fewer tokens per row */
+#define NDL_PREFILL_SPLIT_MIN_KEYS 768   /* 0 bytes for fewer keys per sequence */
 size_t ndl_varlen_prefill_workspace_bytes(int num_seqs, int64_t num_tokens, int max_seqlen,
                                           int max_blocks_per_seq, int num_heads,
                                           int num_kv_heads, int head_dim, int block_size,

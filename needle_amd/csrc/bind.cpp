@@ -178,8 +178,11 @@ PyObject* varlen_prefill(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
   at::Tensor out = at::empty({tokens, heads, d}, q.options());
   size_t need = 0;
-  if (width * c.bs >= NDL_PREFILL_SPLIT_MIN_KEYS)
-    need = p_prefill_workspace((int)seqs, tokens, (int)most, (int)width, (int)heads, (int)hkv,
+  // ops.py's rule: the keys of the longest sequence
+  const int64_t blocks = c.bs > 0 ? (most_ctx + most + c.bs - 1) / c.bs : 0;
+  const int64_t cols = blocks < width ? blocks : width;
+  if (cols * c.bs >= NDL_PREFILL_SPLIT_MIN_KEYS)
+    need = p_prefill_workspace((int)seqs, tokens, (int)most, (int)cols, (int)heads, (int)hkv,
                                (int)d, (int)c.bs, c.code);
   at::Tensor ws;
   if (need) ws = at::empty({(int64_t)need}, q.options().dtype(at::kByte));

@@ -1217,7 +1217,15 @@ NDL_PREFILL_FN(prefill_split_fn, prefill_split_kernel)
 // 2,000 69.2 / 63.6 (31), 100 after 700 31.9 / 29.0 (23).  Once the tiles fill the GPU the
 // clock follows the matrix load and an even split gains nothing (8 x 400 after 4,000, 448
 // tiles: 259 / 236).
+// The longest row is the caller's bound (max_context_len + max_seqlen tokens), not the table's
+// width: a short prompt in a table of the model's length has nothing to split (14/2 heads of 64,
+// 300 tokens, 128 columns, with its append: whole 17.7 us, split 29.1; 32/8 of 128 21.9 / 36.1).
 constexpr int kPrefSplitGain = 40;
+inline int64_t longest_tiles(int max_blocks_per_seq, int block_size, int max_context_len,
+                             int max_seqlen) {
+  const int64_t blocks = ((int64_t)max_context_len + max_seqlen + block_size - 1) / block_size;
+  return (blocks < max_blocks_per_seq ? blocks : max_blocks_per_seq) << block_tile_shift(block_size);
+}
 struct PrefillSplit {
   int64_t takers;
   size_t plan_bytes, ml_bytes, bytes;
@@ -1278,7 +1286,6 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
                               cu_seqlens, context_lens, num_seqs, num_tokens, max_seqlen,
                               max_context_len, num_heads, num_kv_heads, head_dim, block_size,
                               scale, stream);
-  (void)max_context_len;
 
   const int group = num_heads / num_kv_heads;
 
@@ -1325,7 +1332,8 @@ static int launch_prefill(void* out, const void* q, int64_t q_tok_stride, const 
   const bool f16 = dtype_is_f16(dtype);
   PrefillSplit sp;
   if (workspace != nullptr && ((uintptr_t)workspace & 15u) == 0 && !any_scale &&
-      prefill_split(num_seqs, num_tokens, qtiles, num_heads, num_kv_heads, head_dim, a.max_tiles,
+      prefill_split(num_seqs, num_tokens, qtiles, num_heads, num_kv_heads, head_dim,
+                    longest_tiles(max_blocks_per_seq, block_size, max_context_len, max_seqlen),
                     &sp) &&
       workspace_bytes >= sp.bytes) {
     a.takers = (int)sp.takers;

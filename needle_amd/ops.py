@@ -365,6 +365,8 @@ def varlen_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.T
     Equals the reference _prefill_pytorch (attention.py:120-134) when every
     context_lens entry is 0; with a cached prefix the prefix is attended too.
     Returns [num_tokens, num_heads, head_dim].
+    max_context_len bounds context_lens (0: nothing cached).  Results do not depend on it; few
+    tokens after a long prefix are split over the GPU only where it says so.
     With cos/sin ([T, D] rows of the packed tokens), q is the raw projection and each row
     is rotated inside the kernel (ndl_rope_varlen_prefill): the output is bit-identical to
     rope_kv_append's rotated q fed to this function, with k already rotated in the cache
@@ -421,10 +423,11 @@ def varlen_prefill(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.T
             float(scale))
     # few query tiles over many keys: split over workgroups, the pieces in a workspace
     need = 0
-    if block_table.shape[1] * bs >= _lib.NDL_PREFILL_SPLIT_MIN_KEYS:
+    blocks = min(block_table.shape[1], -(-(int(max_context_len) + int(max_seqlen)) // max(bs, 1)))
+    if blocks * bs >= _lib.NDL_PREFILL_SPLIT_MIN_KEYS:
         need = lib.ndl_varlen_prefill_workspace_bytes(
-            n_seqs, n_tok, int(max_seqlen), block_table.shape[1], num_heads, num_kv_heads,
-            head_dim, bs, _DTYPES[q.dtype])
+            n_seqs, n_tok, int(max_seqlen), blocks, num_heads, num_kv_heads, head_dim, bs,
+            _DTYPES[q.dtype])
     if need:
         ws = torch.empty(need, dtype=torch.uint8, device=dev)
         rc = lib.ndl_varlen_prefill_split(out.data_ptr(), q.data_ptr(), qs, _ptr(cos), _ptr(sin),

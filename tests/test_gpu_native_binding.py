@@ -93,10 +93,10 @@ def test_append_and_prefill(native, monkeypatch, dtype):
         return pool
 
     def prefill(q=q, table=table, cu=cu, lens=lens, most=33, scale=0.125, cos=cos, sin=sin, h=h):
-        return ops.varlen_prefill(q, pool0, table, cu, lens, most, scale, h, hkv, d, cos=cos,
-                                  sin=sin)
+        return ops.varlen_prefill(q, pool0, table, cu, lens, most, scale, h, hkv, d,
+                                  max_context_len=900, cos=cos, sin=sin)
     assert native.rope_kv_append(k, v, cos, sin, pool0.clone(), table, lens, cu)
-    assert native.varlen_prefill(q, pool0, table, cu, lens, 33, 0.125, h, hkv, d, 0, cos,
+    assert native.varlen_prefill(q, pool0, table, cu, lens, 33, 0.125, h, hkv, d, 900, cos,
                                  sin) is not None
     changes = [dict(), dict(cos=cos[:5]), dict(cos=cos.double()), dict(sin=sin.cpu()),
                dict(table=table.long()), dict(lens=lens[:2]), dict(cu=cu[:3]),

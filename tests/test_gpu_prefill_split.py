@@ -79,13 +79,13 @@ def _check(name, rope, scale):
     lib = _lib.load()
     code = {torch.bfloat16: 0, torch.float16: 1}[dtype]
     assert lib.ndl_varlen_prefill_workspace_bytes(n_seq, total, max(new), width, h, hkv, d, bs, code)
-    got = ops.varlen_prefill(q, pool, table, cu, lens, max(new), scale, h, hkv, d, cos=cos,
-                             sin=sin)
+    got = ops.varlen_prefill(q, pool, table, cu, lens, max(new), scale, h, hkv, d,
+                             max_context_len=max(max(ctx), 0), cos=cos, sin=sin)
     whole = torch.empty_like(got)
     rc = lib.ndl_varlen_prefill_split(
         whole.data_ptr(), q.data_ptr(), h * d, cos.data_ptr() if rope else None,
         sin.data_ptr() if rope else None, d, pool.data_ptr(), nb, table.data_ptr(), width, width,
-        cu.data_ptr(), lens.data_ptr(), n_seq, total, max(new), 0, h, hkv, d, bs, code,
+        cu.data_ptr(), lens.data_ptr(), n_seq, total, max(new), max(max(ctx), 0), h, hkv, d, bs, code,
         scale, None, 0, torch.cuda.current_stream().cuda_stream)
     assert rc == 0
     torch.cuda.synchronize()
@@ -114,3 +114,37 @@ def test_split_equals_whole_tiles(name, rope):
                                        ("short-table", True)])
 def test_scale_of_any_sign(name, rope, scale):
     _check(name, rope, scale)
+
+
+# The choice counts the keys a sequence can have (max_context_len + max_seqlen), not the table's
+# columns: a short prompt in a table of the model's length runs as in a tight one, without the
+# pieces' workspace; with the bound of a long prefix the pieces are there.
+@pytest.mark.parametrize("native", [True, False])
+def test_wide_table_is_not_a_long_prompt(monkeypatch, native):
+    _lib.load()
+    if not native:
+        monkeypatch.setattr(_lib, "NATIVE", None)
+    h, hkv, d, bs, n, wide = 14, 2, 64, 16, 301, 256
+    g = torch.Generator(device=DEV).manual_seed(3)
+    pool = torch.randn(2, wide, hkv, bs, d, generator=g, device=DEV).to(torch.bfloat16)
+    q = torch.randn(n, h, d, generator=g, device=DEV).to(torch.bfloat16)
+    table = torch.randperm(wide, generator=torch.Generator().manual_seed(5)).to(torch.int32)
+    table = table.view(1, wide).to(DEV)
+    lens = torch.zeros(1, dtype=torch.int32, device=DEV)
+    cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+
+    def run(table, cached):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        out = ops.varlen_prefill(q, pool, table, cu, lens, n, d ** -0.5, h, hkv, d,
+                                 max_context_len=cached)
+        return out, torch.cuda.max_memory_allocated() - before
+    tight, _ = run(table[:, :19].contiguous(), 0)
+    out, used = run(table, 0)
+    assert torch.equal(out, tight) and used < 2 * out.numel() * 2
+    _, used = run(table, 3700)
+    assert used > 16 << 20
+    with pytest.raises(_lib.NeedleAmdError):   # an empty block: the launch's own error
+        ops.varlen_prefill(q, pool[:, :, :, :0], table, cu, lens, n, d ** -0.5, h, hkv, d)
