@@ -222,16 +222,19 @@ def write_kv(k, v, kv_cache, block_table, cu_seqlens, context_lens) -> None:
 def decode_workspace_bytes(num_seqs: int, num_heads: int, num_kv_heads: int, head_dim: int,
                            max_blocks_per_seq: int, block_size: int = 16,
                            partition_tokens: int = 0, dtype: Optional[torch.dtype] = None) -> int:
-    """Bytes of the workspace paged_decode uses for this shape (dtype: of the pool; float32's
-    split has a size of its own)."""
-    if dtype == torch.float32 and partition_tokens == 0:
-        need = int(_lib.load().ndl_paged_decode_f32_workspace_bytes(
+    """Bytes of the workspace paged_decode uses for this shape: for a pool of dtype (float32's
+    split has a size of its own), or, without one, enough for any."""
+    lib = _lib.load()
+    f32 = 0
+    if dtype in (None, torch.float32) and partition_tokens == 0:
+        f32 = int(lib.ndl_paged_decode_f32_workspace_bytes(
             num_seqs, num_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size))
-        if need:   # 0: a shape the launch refuses, sized (and refused) as the other formats'
-            return need
-    return int(_lib.load().ndl_paged_decode_workspace_bytes(
+        if f32 and dtype is not None:
+            return f32   # 0: a shape the launch refuses, sized (and refused) as the other formats'
+    need = int(lib.ndl_paged_decode_workspace_bytes(
         num_seqs, num_heads, num_kv_heads, head_dim, max_blocks_per_seq, block_size,
         partition_tokens))
+    return max(need, f32) if need else 0
 
 
 def paged_decode(q: torch.Tensor, kv_cache: torch.Tensor, block_table: torch.Tensor,
