@@ -584,9 +584,25 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 
 
 # Rows up to which ndl_skinny_linear runs a projection: past them (more than four 16-row
-# tiles) its activations outweigh the weights it streams and the library's GEMM takes over
-# (64 rows, Qwen2-7B gate/up: 69 against 68 us; 32 rows: 60 against 61; 9 rows: 46 against 60).
+# tiles) its activations outweigh the weights it streams and the library's GEMM takes over.
 SKINNY_ROWS = 64
+
+
+def _skinny_rows(n: int, k: int) -> int:
+    """The rows up to which the kernel is the faster one for a single output of n columns.  Past
+    16,384 columns the library streams large weights as fast, and the kernel's re-read of the
+    activations shows from the third 16-row tile on (us, here / library, at 32, 48 and 64 rows:
+    152,064 x 3,584 222 / 264, 221 / 203, 242 / 210; 18,944 x 3,584 31.2 / 33.1, 37.6 / 34.3,
+    41.2 / 35.1; 128,256 x 4,096 210 / 205, 210 / 215, 228 / 218), at short k from the fourth
+    (151,936 x 896 58 / 66, 67 / 73, 72.9 / 70.4).  Narrower ones keep all 64 (4,608 x 3,584
+    12.1 / 13.3, 12.7 / 19.6, 14.2 / 19.0; 3,584 x 18,944 41 / 111, 46 / 114, 53 / 92), and so does
+    the gate/up form, which saves the library's second launch (37,888 x 3,584 52.0 / 58.6, 58.6 /
+    61.4, 63.4 / 65.3)."""
+    if n <= 16384 or k <= 512:
+        return SKINNY_ROWS
+    return 48 if k <= 1024 else 32
+
+
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
@@ -608,6 +624,8 @@ def skinny_linear_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[to
     if (weight.dim() != 2 or weight.shape[1] != k or k == 0 or k % 64 or n == 0
             or n % (16 * halves) or k > 1 << 24 or n > 1 << 28 or weight.dtype != dtype
             or weight.device != x.device or not weight.is_contiguous()):
+        return False
+    if halves == 1 and rows > 32 and rows > _skinny_rows(n, k):
         return False
     st = x.stride(0) if rows > 1 else k
     if x.stride(1) != 1 or st < k or st % 8 or st > 1 << 24:

@@ -100,3 +100,17 @@ def test_other_forms_keep_torchs_linear():
     y.float().sum().backward()
     assert wp.grad is not None
     assert (y.float() - lin).norm() <= 1e-2 * lin.norm()
+
+
+# Wide weights go to the library where the kernel's activations outweigh them; results stay
+# F.linear's on both sides of the line.
+@pytest.mark.parametrize("n,k,last", [(16384, 2048, 64), (16400, 2048, 32), (16400, 1024, 48),
+                                      (16400, 512, 64)])
+def test_rows_by_width(n, k, last):
+    x, w, _ = _inputs(64, n, k, torch.bfloat16, 4)
+    for rows in (32, last, min(last + 1, 64)):
+        assert ops.skinny_linear_takes(x[:rows], w, None) == (rows <= last)
+        assert ops.skinny_linear_takes(x[:rows], w[:16384], None, 2)
+        mag = x[:rows].double().abs() @ w.double().abs().t()
+        _check(ops.linear(x[:rows], w), x[:rows].double() @ w.double().t(), mag, k,
+               torch.bfloat16)
