@@ -43,7 +43,7 @@ class MLP(nn.Module):
         if (self._gate_up is not None and ops.skinny_linear_takes(x, self._gate_up[0], None, 2)
                 and _still_fused(self._gate_up, mods)):
             # a decode step: both projections and their product in one kernel
-            return self.down_proj(ops.linear_silu(x, self._gate_up[0]))
+            return self.down_proj(ops.skinny_linear_silu(x, self._gate_up[0]))
         gate, up = fused_outputs(self._gate_up, mods, x)
         if x.is_cuda:   # one HIP kernel, torch's roundings
             shape = gate.shape

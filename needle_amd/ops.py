@@ -621,11 +621,13 @@ def skinny_linear_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[to
         return False
     rows, k = x.shape
     n = weight.shape[0]
-    if (weight.dim() != 2 or weight.shape[1] != k or k == 0 or k % 64 or n == 0
-            or n % (16 * halves) or k > 1 << 24 or n > 1 << 28 or weight.dtype != dtype
+    if (weight.layout != torch.strided or weight.dim() != 2 or weight.shape[1] != k or k == 0
+            or k % 64 or n == 0 or n % (16 * halves) or k > 1 << 24 or n > 1 << 28 or weight.dtype != dtype
             or weight.device != x.device or not weight.is_contiguous()):
         return False
     if halves == 1 and rows > 32 and rows > _skinny_rows(n, k):
+        return False
+    if not _plain_call():   # before any address: a transform's tensors have none
         return False
     st = x.stride(0) if rows > 1 else k
     if x.stride(1) != 1 or st < k or st % 8 or st > 1 << 24:
@@ -640,14 +642,22 @@ def skinny_linear_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[to
 
 
 def _plain(t: torch.Tensor) -> bool:
-    """An ordinary tensor in an ordinary call: nothing records, traces or transforms it."""
+    """An ordinary tensor that nothing records."""
     return (type(t) in _TENSORS and not (t.requires_grad and torch.is_grad_enabled())
-            and not t.is_conj() and not t.is_neg()
-            and forward_ad._current_level < 0
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._len_torch_function_stack() == 0
-            and not torch.jit.is_tracing())
+            and not t.is_conj() and not t.is_neg())
+
+
+def _plain_call() -> bool:
+    """An ordinary call: nothing differentiates, traces, transforms or intercepts it.  torch
+    has no public names for most of these; where one is missing the answer is no."""
+    try:
+        return (forward_ad._current_level < 0
+                and torch._C._functorch.peek_interpreter_stack() is None
+                and torch._C._len_torch_dispatch_stack() == 0
+                and torch._C._len_torch_function_stack() == 0
+                and not torch.jit.is_tracing())
+    except AttributeError:
+        return False
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor,
@@ -672,9 +682,15 @@ def linear_silu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     the gate rows and then the up rows: linear followed by silu_mul, with the same roundings,
     in one kernel on the rows skinny_linear_takes(x, weight, None, halves=2) accepts."""
     inter = weight.shape[0] // 2
-    if not skinny_linear_takes(x, weight, None, halves=2):
-        gate_up = F.linear(x, weight)
-        return silu_mul(gate_up[:, :inter], gate_up[:, inter:])
+    if skinny_linear_takes(x, weight, None, halves=2):
+        return skinny_linear_silu(x, weight)
+    gate_up = F.linear(x, weight)
+    return silu_mul(gate_up[:, :inter], gate_up[:, inter:])
+
+
+def skinny_linear_silu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """linear_silu's kernel, for a caller that has asked skinny_linear_takes(.., halves=2)."""
+    inter = weight.shape[0] // 2
     rows, k = x.shape
     out = torch.empty((rows, inter), dtype=x.dtype, device=x.device)
     rc = _lib.load().ndl_skinny_linear_silu(

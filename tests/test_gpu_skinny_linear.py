@@ -10,6 +10,9 @@ fp16).
 import pytest
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from needle_amd import ops
 
@@ -114,3 +117,53 @@ def test_rows_by_width(n, k, last):
         mag = x[:rows].double().abs() @ w.double().abs().t()
         _check(ops.linear(x[:rows], w), x[:rows].double() @ w.double().t(), mag, k,
                torch.bfloat16)
+
+
+class _Calls(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen = getattr(self, "seen", 0) + 1
+        return func(*args, **(kwargs or {}))
+
+
+class _Functions(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen = getattr(self, "seen", 0) + (func is F.linear)
+        return func(*args, **(kwargs or {}))
+
+
+# What looks at the operation gets torch's own call, on tensors the kernel would take: a raw
+# launch would lose the tangent, the traced node, the batch dimension, the mode's call.
+@pytest.mark.parametrize("form", ["vmap", "dual", "trace", "dispatch", "function", "inference"])
+def test_forms_of_a_call(form):
+    x, w, b = _inputs(9, 64, 128, torch.bfloat16, 5)
+    assert ops.skinny_linear_takes(x, w, b)
+    takes, want = [], F.linear(x, w, b)
+
+    def call(x):
+        takes.append(ops.skinny_linear_takes(x, w, b))
+        return ops.linear(x, w, b)
+    if form == "vmap":
+        xs = torch.stack([x, 2 * x])
+        got, want = torch.func.vmap(call)(xs), torch.func.vmap(lambda x: F.linear(x, w, b))(xs)
+    elif form == "dual":
+        with forward_ad.dual_level():
+            d = forward_ad.make_dual(x, torch.ones_like(x))
+            got = forward_ad.unpack_dual(call(d)).tangent
+            want = forward_ad.unpack_dual(F.linear(d, w, b)).tangent
+    elif form == "trace":
+        traced = torch.jit.trace(call, (x,), check_trace=False)
+        y = torch.randn_like(x)
+        got, want = traced(y), F.linear(y, w, b)
+    elif form == "inference":     # not one of them: an ordinary call
+        with torch.inference_mode():
+            got = call(x)
+        assert takes == [True]
+        assert (got.float() - want.float()).norm() <= 1e-2 * want.float().norm()
+        return
+    else:
+        with (_Calls() if form == "dispatch" else _Functions()) as mode:
+            got = call(x)
+        assert mode.seen >= 1
+    assert takes and not any(takes)
+    assert got.shape == want.shape and torch.equal(got, want)
+    assert not ops.skinny_linear_takes(x, w.to_sparse_csr(), None)

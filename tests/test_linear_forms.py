@@ -8,6 +8,7 @@ import torch
 import torch.nn as nn
 from torch.autograd import forward_ad
 
+from needle_amd import ops
 from needle_amd.layers.linear import Linear
 
 
@@ -43,3 +44,13 @@ def test_transforms(pair):
     assert torch.equal(a.tangent, b.tangent)
     assert torch.equal(torch.fx.symbolic_trace(ours)(x), theirs(x))
     assert torch.equal(torch.jit.trace(ours, (x,))(x), theirs(x))
+
+
+@pytest.mark.parametrize("owner,name", [(torch._C._functorch, "peek_interpreter_stack"),
+                                        (torch._C, "_len_torch_dispatch_stack"),
+                                        (torch._C, "_len_torch_function_stack"),
+                                        (forward_ad, "_current_level")])
+def test_a_missing_private_name_means_torchs_own(monkeypatch, owner, name):
+    assert ops._plain_call()
+    monkeypatch.delattr(owner, name)
+    assert not ops._plain_call()
