@@ -63,7 +63,8 @@ extern "C" {
 /* Same object as hipStream_t; declared here so callers need no HIP headers. */
 typedef struct ihipStream_t* ndl_stream_t;
 
-#define NDL_ABI_VERSION 8
+/* 9: the float32 decode, prefill split and few-row linear entry points. */
+#define NDL_ABI_VERSION 9
 
 enum ndl_status {
   NDL_OK = 0,

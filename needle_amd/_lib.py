@@ -16,7 +16,7 @@ import torch  # noqa: F401  (loads torch's HIP runtime before ours)
 _PKG_DIR = Path(__file__).resolve().parent
 LIB_PATH = _PKG_DIR / "libneedle_amd.so"
 
-NDL_ABI_VERSION = 8
+NDL_ABI_VERSION = 9
 NDL_DECODE_STATIC_SCRATCH_BYTES = 16 << 20
 NDL_PREFILL_SPLIT_MIN_KEYS = 768
 NDL_DTYPE_BF16 = 0
@@ -201,13 +201,13 @@ def load() -> ctypes.CDLL:
             f"{path} not found: build it with `make -C needle_amd/csrc` "
             "(or __graft_entry__.build()); there is no non-HIP fallback")
     lib = ctypes.CDLL(str(path), mode=ctypes.RTLD_GLOBAL)
+    ver = lib.ndl_abi_version()   # first: a library of another version lacks some of the rest
+    if ver != NDL_ABI_VERSION:
+        raise NeedleAmdError(f"{path}: ABI version {ver} != expected {NDL_ABI_VERSION}")
     for name, (res, args) in _SIGNATURES.items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    ver = lib.ndl_abi_version()
-    if ver != NDL_ABI_VERSION:
-        raise NeedleAmdError(f"ABI version {ver} != expected {NDL_ABI_VERSION}")
     _LIB = lib
     _load_native(lib)
     return lib
@@ -220,6 +220,12 @@ def _load_native(lib: ctypes.CDLL) -> None:
     except ImportError as e:
         warnings.warn(f"needle_amd._native not usable ({e}): build it with `make -C "
                       "needle_amd/csrc`; eager launches go through the interpreter until then")
+        NATIVE = None
+        return
+    if _native.torch_version != torch.__version__:   # built against another torch's C++ classes
+        warnings.warn(f"needle_amd._native was built for torch {_native.torch_version}, this is "
+                      f"{torch.__version__}: run `make -C needle_amd/csrc` again; eager launches "
+                      "go through the interpreter until then")
         NATIVE = None
         return
     _native.init({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value

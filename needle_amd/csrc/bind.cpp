@@ -322,4 +322,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__native() {
+  PyObject* const m = PyModule_Create(&module);
+  // the torch these bindings' inlined code and class layouts are of
+  if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", NDL_TORCH_VERSION) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}
