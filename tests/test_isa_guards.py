@@ -2,7 +2,8 @@
 
 varlen_prefill issues its direct global->LDS loads from inline asm that writes
 M0; M0 is reserved, so the compiler cannot be told about the clobber.  That is
-sound only while nothing else in the prefill kernels uses M0.
+sound only while nothing else in the prefill kernels (of whole tiles, of split
+ones, of scales of 0 or less) uses M0.
 
 RoPE is bit-exact against the reference only while every product and every sum
 is rounded to the element format on its own (needle/layers/attention.py:277-283
@@ -54,9 +55,16 @@ def device_asm(tmp_path_factory):
 
 def test_prefill_kernels_use_m0_only_for_direct_lds_loads(device_asm):
     lines = device_asm("varlen_prefill")
+    # head_dim 64 and 128, with and without RoPE of q, bf16 and fp16, of each launch's kernel
+    names = ("21varlen_prefill_kernel", "20prefill_split_kernel", "24prefill_any_scale_kernel")
     kernels = [i for i, l in enumerate(lines)
-               if re.match(r"_ZN3ndl21varlen_prefill_kernel.*:", l)]
-    assert len(kernels) == 8          # head_dim 64 and 128, with and without RoPE of q, bf16 and fp16
+               if re.match(rf"_ZN3ndl({'|'.join(names)}).*:", l)]
+    assert len(kernels) == 8 * len(names)
+    # and nothing else of the file loads to LDS this way
+    assert sum("global_load_lds" in l and not l.strip().startswith(";") for l in lines) == sum(
+        "global_load_lds" in l and not l.strip().startswith(";") for start in kernels
+        for l in lines[start:next(i for i in range(start, len(lines))
+                                  if lines[i].startswith(".Lfunc_end"))])
     for start in kernels:
         end = next(i for i in range(start, len(lines)) if lines[i].startswith(".Lfunc_end"))
         body = [l.strip() for l in lines[start:end] if not l.strip().startswith(";")]
