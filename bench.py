@@ -91,13 +91,18 @@ def build_workload(torch, wl, device):
 
 ROOT = os.path.dirname(os.path.abspath(__file__))
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "paged_decode_llama3_8b_hbm_traffic.md")
-DECODE_SOURCE = os.path.join(ROOT, "needle_amd", "csrc", "paged_decode.hip")
+# what the counted launch pair is compiled from: the attention, the merge, their helpers
+DECODE_SOURCES = [os.path.join(ROOT, "needle_amd", "csrc", n)
+                  for n in ("paged_decode.hip", "decode_stream.hpp", "ndl_common.hpp")]
 
 
-def source_sha16(path=DECODE_SOURCE):
+def source_sha16(paths=DECODE_SOURCES):
     import hashlib
-    with open(path, "rb") as f:
-        return hashlib.sha256(f.read()).hexdigest()[:16]
+    h = hashlib.sha256()
+    for path in paths:
+        with open(path, "rb") as f:
+            h.update(f.read())
+    return h.hexdigest()[:16]
 
 
 def measured_traffic():
@@ -120,10 +125,10 @@ def measured_traffic():
         return None, "traffic summary has no traffic_bytes_per_launch line"
     now = source_sha16()
     if info.get("kernel_source_sha16") != now:
-        print(f"bench.py: {TRAFFIC_PROFILE} was counted on paged_decode.hip "
+        print(f"bench.py: {TRAFFIC_PROFILE} was counted on decode sources "
               f"{info.get('kernel_source_sha16')}, the source is now {now}: traffic not "
               "reported", file=sys.stderr, flush=True)
-        return None, (f"stale: counted on paged_decode.hip {info.get('kernel_source_sha16')}, "
+        return None, (f"stale: counted on decode sources {info.get('kernel_source_sha16')}, "
                       f"source now {now}")
     return int(info["traffic_bytes_per_launch"]), info.get("kernels", "")
 
