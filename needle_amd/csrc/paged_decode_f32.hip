@@ -87,10 +87,10 @@ __global__ __launch_bounds__(64 * kF32Waves) void paged_decode_f32_kernel(Decode
   const float* const vplane = (const float*)a.vplane;
   __shared__ __attribute__((aligned(16))) float sacc[NW * E * 64];
   __shared__ float sm[NW * 16], sl[NW * 16];
-  // The split form at head_dim 128 has no registers to spare: with its arguments held it spilled
-  // to memory (32 of 1,000 tokens as whole sequences, 28/4 heads: 45.7 us, read again 41.2).
+  // The split form has no registers to spare: with its arguments held it spilled to memory at
+  // head_dim 128 (32 of 1,000 tokens as whole sequences, 28/4 heads: 45.7 us, read again 41.2).
   auto args = [&]() -> decltype(auto) {
-    if constexpr (SPLIT && D == 128)
+    if constexpr (SPLIT)
       return fresh_args();
     else
       return (a);

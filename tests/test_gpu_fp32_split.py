@@ -37,8 +37,12 @@ CASES = {
     "past-short-128": (28, 4, 128, 16, [288, 17, 100, -1], 90),
     "past-even": (32, 8, 128, 16, [640 + i % 9 for i in range(28)] + [1500], 30),
 }
-# never split: rows appended by a launch before (768 workgroups, 64 sequences)
-ONE_LAUNCH = {"append-first": (32, 8, 128, 16, [(7 * i) % 330 for i in range(95)] + [-1], 0),
+# never split: rows appended by a launch before (768 workgroups, 64 sequences); tables of up to
+# 40 and 64 tiles where the pairs fill the GPU once or twice
+ONE_LAUNCH = {"full-once": (28, 4, 128, 16, [639 - 9 * i for i in range(50)], 0),
+              "full-once-64": (14, 2, 64, 32, [1023 - 11 * i for i in range(64)], 0),
+              "full-twice": (32, 32, 128, 16, [1023 - 31 * i for i in range(16)], 0),
+              "append-first": (32, 8, 128, 16, [(7 * i) % 330 for i in range(95)] + [-1], 0),
               "append-first-64": (24, 12, 64, 16, [(11 * i) % 330 for i in range(64)], 0)}
 
 
@@ -107,6 +111,8 @@ def test_vs_float64(name, form):
     q, pool, table, lens, more = _inputs(case, form)
     n, width = table.shape
     nb = pool.shape[1]
+    need = ops.decode_workspace_bytes(n, h, hkv, d, width, bs, 0, torch.float32)
+    assert (need > 256) == (name in CASES)
     got_pool = pool.clone()
     got = ops.paged_decode(q, got_pool, table, lens, d ** -0.5, h, hkv, d, **more)
     want_pool, k, qr = pool.clone(), more.get("new_k"), q
