@@ -277,11 +277,12 @@ __global__ __launch_bounds__(64 * NWK * NWR) __attribute__((amdgpu_waves_per_eu(
 // The split of a workgroup's four waves.  Four over the keys of 16 rows keep the longest row
 // block's chain short, and a small batch's time is that chain; two over the keys of 32 rows
 // read each K/V tile half as often, which a batch that fills the GPU is bound by.  us at
-// 4 x 1 / 2 x 2 (1 x 4, the split before, in brackets): 14/2 heads of 64, prompts of 64 to
-// 1,024 tokens, 2,168 in all, 49.5 / 69 (110); 28/4 of 128, 33 tokens after 2,000 54 / 94
-// (175), 1,000 118 / 121 (110), 6 x 500 199 / 176 (180), 8 x 1,000 979 / 757 (738), 16 x 400
-// 376 / 286 (346).  The line: row blocks of 16, scaled by how even the prompts are (a batch
-// of uneven ones is as long as its longest), against 1.5 per SIMD.
+// 4 x 1 / 2 x 2 / 1 x 4 of this kernel, and before it (one wave per 16 rows, every tile masked,
+// first rows first): 14/2 heads of 64, prompts of 64 to 1,024 tokens, 2,168 in all, with the
+// append, 49.5 / 69 / - and 110; 28/4 of 128, 33 tokens after 2,000 54 / 94 / 175 and 58, 1,000
+// 118 / 121 / 110 and 153, 6 x 500 199 / 176 / 180 and 311, 8 x 1,000 979 / 757 / 738 and 1,189,
+// 16 x 400 376 / 286 / 346 and 591.  The line: row blocks of 16, scaled by how even the prompts
+// are (a batch of uneven ones is as long as its longest), against 1.5 per SIMD.
 constexpr double kPrefF32Blocks = 1536;
 
 template <int NWK, int NWR>
