@@ -177,8 +177,9 @@ size_t ndl_paged_decode_f32_workspace_bytes(int num_seqs, int num_heads, int num
  * (k, v, cos and sin NULL), ndl_paged_decode_append (cos and sin NULL) or
  * ndl_rope_paged_decode_append give for NDL_DTYPE_F32, up to the order of the fp32 sums.  With
  * a 16-byte aligned workspace of ndl_paged_decode_f32_workspace_bytes (calls that share one
- * must not overlap) sequences are split over workgroups and merged; with none, or a smaller
- * one, each (kv head, sequence) is one workgroup, as in those entry points.
+ * must not overlap) sequences are split over workgroups and merged where their lengths gain by
+ * it; with none, or a smaller one, each (kv head, sequence) is one workgroup, as in those entry
+ * points.
  *
  * Replaces: needle/layers/attention.py:140-159, :291-310 in a float32 model.
  */
