@@ -829,7 +829,7 @@ def main():
             "traffic_kernels": traffic_kernels,
             "traffic_source": "profiles/paged_decode_llama3_8b_hbm_traffic.md (rocprofv3 "
                               "FETCH_SIZE x2 + WRITE_SIZE x1 per launch pair, scaled by a "
-                              "1 GiB copy; keyed to the hash of paged_decode.hip)",
+                              "1 GiB copy; keyed to the hash of the pair's sources)",
             "kernel": "the timed step's launch pair per layer: fused append + paged decode "
                       "attention (ndl_paged_decode_append) and the partition merge",
             "algorithmic_bytes_per_launch": dec_b + app_b, "avg_launch_us": round(pair_us, 2),
